@@ -88,7 +88,7 @@ int launch_pbs1(fhe_ctx *ctx, const uint32_t *in, const uint32_t *tv, int tv_str
         int rc = prepare_pbs1(ctx, s);
         if (rc) return rc;
         HIP_TRY(launch_blind_rotate1w2(in, n0, ctx->bk1w2, tv, tv_stride, out, se, B, s),
-                "pbs lvl01 (two waves per ciphertext)");
+                "pbs lvl01 (two waves per polynomial)");
         return FHE_OK;
     }
     HIP_TRY(launch_blind_rotate1(in, n0, ctx->bk1, tv, tv_stride, out, se, B, s), "pbs lvl01");

@@ -27,7 +27,7 @@ struct fhe_ctx {
     // upload) and its tables
     float *bk1m = nullptr;  // [i][row][col][limb][512 complex] FP32
     bool bk1m_valid = false;
-    // two-waves-per-ciphertext kernel: bk1 permuted into its order (rebuilt
+    // two-waves-per-polynomial kernel: bk1 permuted into its order (rebuilt
     // on demand, bk1w2_valid cleared by every lvl1 key upload)
     fhe::cd *bk1w2 = nullptr;
     bool bk1w2_valid = false;
@@ -85,9 +85,11 @@ inline hipStream_t pick(fhe_ctx *ctx, void *stream)
     return stream ? static_cast<hipStream_t>(stream) : ctx->stream;
 }
 
-// untuned: batches below this many ciphertexts use two waves per ciphertext
-// (one MI355X, n0 = 636: two waves 4.40 / 5.79 / 6.24 ms at 256 / 512 / 768
-// ciphertexts, one wave 5.17 / 5.41 / 5.94)
+// untuned: batches below this many ciphertexts use two waves per polynomial
+// and a compute unit per ciphertext (one MI355X, n0 = 672: 2.4 ms up to 256
+// ciphertexts, 4.9 from 257, where a second round starts; one wave per
+// ciphertext, n0 = 636, 5.17 / 5.41 / 5.94 ms at 256 / 512 / 768).  The two kernels sum in different
+// orders, so moving the line would change the words that a batch returns.
 constexpr int kPbs1TwoWaveBelow = 512;
 
 // set on this thread between fhe_graph_begin and fhe_graph_end: scratch
@@ -147,7 +149,7 @@ inline int iks_tile(const fhe_ctx *ctx, int kind, int B)
     return tuned(ctx, kind == 10 ? FHE_TUNE_IKS_SPLIT : FHE_TUNE_IKS20_SPLIT, B, 8);
 }
 
-// waves per ciphertext of the FP64 lvl1 blind rotation for a batch of B
+// waves per polynomial of the FP64 lvl1 blind rotation for a batch of B
 inline int pbs1_waves(const fhe_ctx *ctx, int B)
 {
     return tuned(ctx, FHE_TUNE_PBS1_WAVES, B, B < kPbs1TwoWaveBelow ? 2 : 1);

@@ -422,12 +422,10 @@ __device__ __forceinline__ void transpose_reg_lane_hi_lds(cd v[4], cd *tile, int
 // lane-bits-4-5 transpose (PERM: lane swaps; otherwise through the tile),
 // the other two go through a wave-private LDS tile of kLaneTile double2
 // (row strides 20 and 5, conflict-free for 16-lane b128 accesses).  The
-// swaps move VALU work in for LDS traffic out, which pays on short launches
-// and costs on long ones: the kernels that use this transform instantiate
-// both forms and pick one by batch size (both move the same words, so the
-// results are identical).  t64 = W64^(lane & 15),
-// t16 = W16^(lane & 3).  Input: register r, lane L holds x_r[L]; output:
-// register q, lane l holds X_r[m] for r = l >> 4,
+// swaps move VALU work in for LDS traffic out, which pays in the blind
+// rotations; both forms move the same words, so the results are identical.
+// t64 = W64^(lane & 15), t16 = W16^(lane & 3).  Input: register r, lane L
+// holds x_r[L]; output: register q, lane l holds X_r[m] for r = l >> 4,
 // m = ((l >> 2) & 3) + 4 (l & 3) + 16 q.
 template <bool PERM>
 __device__ __forceinline__ void lanes64_fwd(cd v[4], cd *tile, int l, cd t64, cd t16)

@@ -1,14 +1,14 @@
-// pbs_lvl1w2.hip -- lvl1 blind rotation with two waves per ciphertext, for
-// batches too small to fill the GPU with one wave per ciphertext.
+// pbs_lvl1w2.hip -- lvl1 blind rotation with two waves per polynomial and the
+// digit rows side by side, for batches too small to fill the GPU with one
+// wave per ciphertext.
 //
 // Same computation as k_blind_rotate1 (pbs_lvl1.hip; TFHEpp BlindRotate,
 // gatebootstrapping.hpp:15-43, CMUX detwfa.cpp:21-30, external product
-// trgsw.cpp:78-103), split over two waves: each wave owns 256 of the 512
-// complex points of every polynomial (4 per lane), so a ciphertext's CMUX
-// step runs on two SIMDs and a small batch finishes in about half the time.
-// The accumulator stays in LDS (the rotation reads any coefficient); each
-// wave rotates and decomposes its own coefficients, and the transform
-// (512 = 4 x 128) exchanges once between the waves:
+// trgsw.cpp:78-103), with a whole compute unit on one ciphertext: each
+// polynomial is split over two waves (256 of the 512 complex points each, 4
+// per lane), the six digit rows of a CMUX step are transformed at once by
+// twelve waves, and four more carry the two accumulator columns back.  The
+// transform (512 = 4 x 128) exchanges once between its two waves:
 //   step A (registers): u_k[n0] = w^(n0 (4k+1)) sum_p c_p z[n0 + 128 p] i^(pk),
 //           c_p = exp(i pi p / 8), n0 = lane + 64 wave < 128, k < 4;
 //   exchange: wave v takes u_k for k = 2v, 2v+1 (all 128 n0);
@@ -29,7 +29,6 @@ namespace {
 constexpr int N1 = Lvl1::N;
 constexpr int kPolyW = 512;  // complex points per polynomial
 constexpr uint32_t kDecOffW = decomp_total_offset<uint32_t, 32, Lvl1::l, Lvl1::Bgbit>();
-constexpr uint32_t kDigitFlipW = (1u << 31) | (1u << 25) | (1u << 19);
 
 // natural frequency of (wave, lane, register) in the output layout
 __host__ __device__ constexpr int f1w(int w, int l, int q)
@@ -62,12 +61,12 @@ __device__ __forceinline__ cd c8w(int p)
     return p == 1 ? cd{c1, s1} : p == 2 ? cd{kR2, kR2} : cd{s1, c1};
 }
 
-// Forward transform.  xch: the workgroup's 2 x kLaneTile double2, the two
-// wave tiles; the exchange puts wave v's two sequences (k = 2v, 2v + 1) at
-// the start of v's own tile, so after the exchange a wave touches only its
-// own tile until the next exchange.
-template <bool PERM>
-__device__ __forceinline__ void fft512w_fwd(cd v[4], cd *xch, int lane, int wave, const TwW &tw)
+// The forward transform of one wave's half, in two parts around the exchange
+// between the two halves (the caller's barrier).  pair: the two halves' tiles
+// (2 x kLaneTile double2); part A puts sequence k of half v = k >> 1 at the
+// start of v's tile, part C goes on in the half's own tile, which no other
+// wave touches until the next exchange.
+__device__ __forceinline__ void fft512w_fwd_a(cd v[4], cd *pair, int lane, int half, const TwW &tw)
 {
     v[1] = cmul(v[1], c8w(1));
     v[2] = cmul(v[2], c8w(2));
@@ -81,33 +80,30 @@ __device__ __forceinline__ void fft512w_fwd(cd v[4], cd *xch, int lane, int wave
             if (k < 3) g = cmul(g, tw.rho);
         }
     }
-    const int n0 = lane + 64 * wave;
-    __syncthreads();  // both waves have left their tiles
+    const int n0 = lane + 64 * half;
 #pragma unroll
-    for (int k = 0; k < 4; k++) xch[(k >> 1) * kLaneTile + (k & 1) * 128 + n0] = v[k];
-    __syncthreads();
+    for (int k = 0; k < 4; k++) pair[(k >> 1) * kLaneTile + (k & 1) * 128 + n0] = v[k];
+}
+
+__device__ __forceinline__ void fft512w_fwd_c(cd v[4], cd *tile, int lane, const TwW &tw)
+{
 #pragma unroll
-    for (int j = 0; j < 4; j++) v[j] = xch[wave * kLaneTile + (j >> 1) * 128 + lane + 64 * (j & 1)];
+    for (int j = 0; j < 4; j++) v[j] = tile[(j >> 1) * 128 + lane + 64 * (j & 1)];
 #pragma unroll
     for (int s = 0; s < 2; s++) {
         const cd a = v[2 * s], b = v[2 * s + 1];
         v[2 * s] = cadd(a, b);
         v[2 * s + 1] = cmul(csub(a, b), tw.t128);
     }
-    lanes64_fwd<PERM>(v, xch + wave * kLaneTile, lane, tw.t64, tw.t16);
+    lanes64_fwd<true>(v, tile, lane, tw.t64, tw.t16);
 }
 
-// Inverse (unnormalised: returns 512 z): frequency layout in, time layout out.
-// The wave writes its exchange words into its own tile, which the other wave
-// does not touch between the last barrier (the forward exchange's second, or
-// the previous inverse's tail) and the reads, so no barrier precedes the
-// write.  TAIL_SYNC: wait for both waves' exchange reads before returning
-// (the caller's next use of its tile would overwrite words the other wave
-// reads); not needed when a workgroup barrier follows anyway.
-template <bool PERM, bool TAIL_SYNC = true>
-__device__ __forceinline__ void fft512w_inv(cd v[4], cd *xch, int lane, int wave, const TwW &tw)
+// The inverse (unnormalised: returns 512 z), frequency layout in, time layout
+// out, in two parts around the exchange: part A ends with the wave's words in
+// its own tile, part C reads both halves' tiles.
+__device__ __forceinline__ void fft512w_inv_a(cd v[4], cd *tile, int lane, const TwW &tw)
 {
-    lanes64_inv<PERM>(v, xch + wave * kLaneTile, lane, tw.t64, tw.t16);
+    lanes64_inv<true>(v, tile, lane, tw.t64, tw.t16);
 #pragma unroll
     for (int s = 0; s < 2; s++) {
         const cd a = v[2 * s], b = cmulc(v[2 * s + 1], tw.t128);
@@ -115,12 +111,15 @@ __device__ __forceinline__ void fft512w_inv(cd v[4], cd *xch, int lane, int wave
         v[2 * s + 1] = csub(a, b);
     }
 #pragma unroll
-    for (int j = 0; j < 4; j++) xch[wave * kLaneTile + (j >> 1) * 128 + lane + 64 * (j & 1)] = v[j];
-    __syncthreads();
-    const int n0 = lane + 64 * wave;
+    for (int j = 0; j < 4; j++) tile[(j >> 1) * 128 + lane + 64 * (j & 1)] = v[j];
+}
+
+__device__ __forceinline__ void fft512w_inv_c(cd v[4], const cd *pair, int lane, int half,
+                                              const TwW &tw)
+{
+    const int n0 = lane + 64 * half;
 #pragma unroll
-    for (int k = 0; k < 4; k++) v[k] = xch[(k >> 1) * kLaneTile + (k & 1) * 128 + n0];
-    if (TAIL_SYNC) __syncthreads();
+    for (int k = 0; k < 4; k++) v[k] = pair[(k >> 1) * kLaneTile + (k & 1) * 128 + n0];
     {
         cd g = tw.beta;
 #pragma unroll
@@ -135,108 +134,169 @@ __device__ __forceinline__ void fft512w_inv(cd v[4], cd *xch, int lane, int wave
     v[3] = cmulc(v[3], c8w(3));
 }
 
-// (X^a - 1) * poly at coefficient n, a in [0, 2N)
-__device__ __forceinline__ uint32_t rot_minus_one_w(const uint32_t *poly, uint32_t a, int n)
-{
-    const uint32_t idx = (uint32_t(n) - a) & (2u * N1 - 1);
-    uint32_t v = poly[idx & (N1 - 1)];
-    if (idx & N1) v = 0u - v;
-    return v - poly[n];
-}
+constexpr int kRowWaves = 2 * Lvl1::rows;     // two halves per digit row
+constexpr int kColWaves = 4;                  // two halves per accumulator column
+constexpr int kWaves = kRowWaves + kColWaves; // 16: also (column, half, register) of the products
+static_assert(kWaves == 2 * 2 * 4, "one product wave per column, half and register");
 
-// gadget digits (trgsw.cpp:21-39) as one signed field extract of the word
-// prepared with the offset and the flipped top bit of every 6-bit field
-__device__ __forceinline__ uint32_t prep_w(uint32_t x) { return (x + kDecOffW) ^ kDigitFlipW; }
-__device__ __forceinline__ double digit_w(uint32_t u, int d)
-{
-    const int sh = 32 - Lvl1::Bgbit * (d + 1);
-    return double(int32_t(__builtin_amdgcn_sbfe(int32_t(u), sh, Lvl1::Bgbit)));
-}
+// LDS of one blind rotation (106 KB of the CU's 160).  ext holds a column
+// followed by its negation and the column again, so that coefficient n of
+// X^a acc is word ((n - a) mod 2N) + k with the wrap's sign in the data and
+// the lane's eight words at immediate offsets from one base.
+struct alignas(16) Br1wLds {
+    cd row[kRowWaves][kLaneTile];  // row waves' tiles, then their row's spectrum
+    cd col[kColWaves][kLaneTile];  // product sums, then the column waves' tiles
+    uint32_t ext[2][3 * N1];
+    uint32_t step[kMaxN0 + 1];
+    int rank[kWaves];
+};
+static_assert(64 * kWaves >= kMaxN0, "one thread per step");
 
-// three waves per SIMD (168 VGPRs, no spills)
-template <bool PERM>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_blind_rotate1w2(
+// One workgroup of 16 waves per ciphertext, one workgroup per compute unit.
+// A CMUX step, with a barrier after each phase:
+//   1. row waves (12: digit row r, half h) rotate and decompose their own
+//      256 points of the row and run the transform up to its exchange;
+//   2. they finish it and leave the row's spectrum in their tile;
+//   3. all 16 waves form the products: wave (column, half, register) sums
+//      the six rows in row order for its 64 points, with the key words
+//      loaded one step ahead;
+//   4. column waves (4: column, half) run the inverse up to its exchange;
+//   5. they finish it and add it to their words of the accumulator (kept in
+//      registers), writing the three copies the rotation reads.
+// Every value is computed by the same operations in the same order whatever
+// the batch size.
+//
+// Bound by the LDS writes of the row waves (74-80 bytes a clock: phase 2 is
+// 12 waves x 12 KB) and by the chain through the five barriers, about 8,100
+// cycles a step (1,420 / 3,030 / 750 / 1,870 / 1,050 by phase); it is for
+// batches that leave the chip idle.  One MI355X, n0 = 672, up to 256
+// ciphertexts: 2.37-2.5 ms against 4.5-4.6 with the rows one after the other
+// on two waves.  Not kept: the lane exchanges as DPP selects (no LDS traffic,
+// but about 8 cycles an instruction: phase 2 3,950), the first exchange
+// through LDS instead of register swaps (3,970), loading the key words right
+// after the products (96 KB through the 64-byte L1 port: phase 3 1,930).
+__global__ __launch_bounds__(64 * kWaves) void k_blind_rotate1w2(
     const uint32_t *__restrict__ in, int n0, const cd *__restrict__ bk,
     const uint32_t *__restrict__ tv, int tv_stride, uint32_t *__restrict__ out, int sample_extract,
     int B)
 {
-    __shared__ uint32_t acc[2][N1];
-    __shared__ cd xch[2 * kLaneTile];
+    __shared__ Br1wLds lds;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ct = blockIdx.x;
     if (ct >= B) return;
     const uint32_t *c0 = in + size_t(ct) * (n0 + 1);
     const uint32_t *tvp = tv + size_t(ct) * tv_stride;
-    const TwW tw = make_tww(lane, wave);
-    const int nb = lane + 64 * wave;
+    const int half = wave & 1;
+    const TwW tw = make_tww(lane, half);
+    const int nb = lane + 64 * half;
+    const bool is_row = wave < kRowWaves;
+    // row waves: the row's column and digit.  The digit's sign flip is an
+    // addition into its field's top bit (its carry leaves the field upwards):
+    // digit = signed field of (X^a acc - acc) + kd.
+    const int rcol = (wave >> 1) / Lvl1::l, rdig = (wave >> 1) % Lvl1::l;
+    const int sh = 32 - Lvl1::Bgbit * (rdig + 1);
+    const uint32_t kd = kDecOffW + (1u << (sh + Lvl1::Bgbit - 1));
+    // column waves: their column and the words lane + 64 half + 128 p (+ 512)
+    const int col = (wave - kRowWaves) >> 1;
+    uint32_t own[8];
+    auto put = [&](int k) {
+        uint32_t *e = lds.ext[col] + nb + 128 * (k >> 1) + 512 * (k & 1);
+        e[0] = own[k];
+        e[N1] = 0u - own[k];
+        e[2 * N1] = own[k];
+    };
 
     // acc = (0, X^bbar tv), bbar = 2N - (b >> 21)   (no rounding)
-    {
+    if (!is_row) {
         const uint32_t bbar = 2u * N1 - (c0[n0] >> (32 - 1 - Lvl1::nbit));
 #pragma unroll
-        for (int k = 0; k < N1 / 128; k++) {
-            const int n = tid + 128 * k;
+        for (int k = 0; k < 8; k++) {
+            const int n = nb + 128 * (k >> 1) + 512 * (k & 1);
             const uint32_t idx = (uint32_t(n) - bbar) & (2u * N1 - 1);
             const uint32_t v = tvp[idx & (N1 - 1)];
-            acc[0][n] = 0;
-            acc[1][n] = (idx & N1) ? 0u - v : v;
+            own[k] = col == 0 ? 0u : (idx & N1) ? 0u - v : v;
+            put(k);
         }
     }
-    __syncthreads();
 
+    // the steps with a rotation to do (a-bar = 0 is skipped), in order, as
+    // i << 12 | a-bar: thread i ranks its step among the nonzero ones
     constexpr uint32_t kRound = 1u << (32 - 2 - Lvl1::nbit);
-    for (int i = 0; i < n0; i++) {
-        const uint32_t abar = (c0[i] + kRound) >> (32 - 1 - Lvl1::nbit);
-        if (abar == 0) continue;
-        const cd *bki = bk + size_t(i) * (Lvl1::rows * 2 * kPolyW) + wave * 256 + lane;
-        cd fd0[4], fd1[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) fd0[q] = fd1[q] = cd{0.0, 0.0};
-#pragma unroll 1
-        for (int c = 0; c < 2; c++) {
-            // this wave's coefficients of (X^abar - 1) acc_c, prepared for digits
-            uint32_t u[8];
-#pragma unroll
-            for (int p = 0; p < 4; p++) {
-                u[2 * p] = prep_w(rot_minus_one_w(acc[c], abar, nb + 128 * p));
-                u[2 * p + 1] = prep_w(rot_minus_one_w(acc[c], abar, nb + 128 * p + 512));
-            }
-#pragma unroll 1
-            for (int d = 0; d < Lvl1::l; d++) {
-                const int r = c * Lvl1::l + d;
-                // key words requested before the transform
-                cd b0[4], b1[4];
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    b0[q] = bki[r * 2 * kPolyW + q * 64];
-                    b1[q] = bki[r * 2 * kPolyW + kPolyW + q * 64];
-                }
-                cd v[4];
-#pragma unroll
-                for (int p = 0; p < 4; p++) v[p] = cd{digit_w(u[2 * p], d), digit_w(u[2 * p + 1], d)};
-                fft512w_fwd<PERM>(v, xch, lane, wave, tw);
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    cmac(fd0[q], v[q], b0[q]);
-                    cmac(fd1[q], v[q], b1[q]);
-                }
-            }
+    {
+        const uint32_t abar = tid < n0 ? (c0[tid] + kRound) >> (32 - 1 - Lvl1::nbit) : 0u;
+        const uint64_t some = __ballot(abar != 0);
+        if (lane == 0) lds.rank[wave] = __popcll(some);
+        __syncthreads();
+        int at = 0, all = 0;
+        for (int w = 0; w < kWaves; w++) {
+            if (w == wave) at = all;
+            all += lds.rank[w];
         }
-        // both waves' rotation reads of acc are complete (the transforms
-        // synchronised them); each wave updates only its own coefficients
-        fft512w_inv<PERM>(fd0, xch, lane, wave, tw);
+        if (abar) lds.step[at + __popcll(some & ((1ull << lane) - 1))] = uint32_t(tid) << 12 | abar;
+        if (tid == 0) lds.step[all] = 0;
+    }
+    // product wave: column, and slot (half, register) of 64 points
+    const int pcol = wave >> 3, slot = wave & 7;
+    cd key[Lvl1::rows];
+    auto load_key = [&](uint32_t step) {
+        const cd *k = bk + (size_t(step >> 12) * Lvl1::rows * 2 + pcol) * kPolyW + slot * 64 + lane;
 #pragma unroll
-        for (int p = 0; p < 4; p++) {
-            acc[0][nb + 128 * p] += trunc_torus32(fd0[p].x);
-            acc[0][nb + 128 * p + 512] += trunc_torus32(fd0[p].y);
+        for (int r = 0; r < Lvl1::rows; r++) key[r] = k[r * 2 * kPolyW];
+    };
+    __syncthreads();
+    uint32_t step = __builtin_amdgcn_readfirstlane(lds.step[0]);
+    if (step) load_key(step);
+
+    for (int k = 1; step; k++) {
+        const uint32_t ahead = lds.step[k];
+        cd v[4];
+        if (is_row) {
+            const uint32_t *rot = lds.ext[rcol] + ((uint32_t(nb) - step) & (2u * N1 - 1));
+            const uint32_t *neg = lds.ext[rcol] + N1 + nb;
+            double x[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const int o = 128 * (k >> 1) + 512 * (k & 1);
+                x[k] = double(int32_t(__builtin_amdgcn_sbfe(int32_t(rot[o] + neg[o] + kd), sh, Lvl1::Bgbit)));
+            }
+#pragma unroll
+            for (int p = 0; p < 4; p++) v[p] = cd{x[2 * p], x[2 * p + 1]};
+            fft512w_fwd_a(v, lds.row[wave & ~1], lane, half, tw);
         }
-        // the step's closing barrier follows this transform's exchange reads
-        fft512w_inv<PERM, false>(fd1, xch, lane, wave, tw);
+        __syncthreads();
+        if (is_row) {
+            fft512w_fwd_c(v, lds.row[wave], lane, tw);
 #pragma unroll
-        for (int p = 0; p < 4; p++) {
-            acc[1][nb + 128 * p] += trunc_torus32(fd1[p].x);
-            acc[1][nb + 128 * p + 512] += trunc_torus32(fd1[p].y);
+            for (int q = 0; q < 4; q++) lds.row[wave][q * 64 + lane] = v[q];
+        }
+        __syncthreads();
+        {
+            cd fd{0.0, 0.0};
+#pragma unroll
+            for (int r = 0; r < Lvl1::rows; r++)
+                cmac(fd, lds.row[2 * r + (slot >> 2)][(slot & 3) * 64 + lane], key[r]);
+            lds.col[2 * pcol + (slot >> 2)][(slot & 3) * 64 + lane] = fd;
+        }
+        __syncthreads();
+        if (!is_row) {
+            cd *tile = lds.col[wave - kRowWaves];
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[q] = tile[q * 64 + lane];
+            wave_lds_sync();
+            fft512w_inv_a(v, tile, lane, tw);
+        }
+        // the next step's key words, in flight until its products
+        step = __builtin_amdgcn_readfirstlane(ahead);
+        if (step) load_key(step);
+        __syncthreads();
+        if (!is_row) {
+            fft512w_inv_c(v, lds.col[2 * col], lane, half, tw);
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                own[k] += trunc_torus32(k & 1 ? v[k >> 1].y : v[k >> 1].x);
+                put(k);
+            }
         }
         __syncthreads();
     }
@@ -244,19 +304,12 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     if (sample_extract) {
         // SampleExtractIndex 0: out[0] = acc0[0], out[n] = -acc0[N - n], out[N] = acc1[0]
         uint32_t *o = out + size_t(ct) * (N1 + 1);
-#pragma unroll
-        for (int k = 0; k < N1 / 128; k++) {
-            const int n = tid + 128 * k;
-            o[n] = n == 0 ? acc[0][0] : 0u - acc[0][N1 - n];
-        }
-        if (tid == 0) o[N1] = acc[1][0];
+        o[tid] = tid == 0 ? lds.ext[0][0] : lds.ext[0][2 * N1 - tid];
+        if (tid == 0) o[N1] = lds.ext[1][0];
     } else {
         uint32_t *o = out + size_t(ct) * 2 * N1;
-#pragma unroll
-        for (int k = 0; k < N1 / 128; k++) {
-            o[tid + 128 * k] = acc[0][tid + 128 * k];
-            o[N1 + tid + 128 * k] = acc[1][tid + 128 * k];
-        }
+        o[tid] = lds.ext[0][tid];
+        o[N1 + tid] = lds.ext[1][tid];
     }
 }
 
@@ -292,14 +345,8 @@ hipError_t launch_blind_rotate1w2(const uint32_t *in, int n0, const cd *bk, cons
                                   hipStream_t s)
 {
     if (B <= 0) return hipSuccess;
-    // the lane transform's first transpose as register swaps: measured A/B
-    // 4.42 against 4.61 ms at 256 ciphertexts, 6.12 against 5.87 ms at 512
-    if (B <= 256)
-        hipLaunchKernelGGL(k_blind_rotate1w2<true>, dim3(B), dim3(128), 0, s, in, n0, bk, tv,
-                           tv_stride, out, int(sample_extract), B);
-    else
-        hipLaunchKernelGGL(k_blind_rotate1w2<false>, dim3(B), dim3(128), 0, s, in, n0, bk, tv,
-                           tv_stride, out, int(sample_extract), B);
+    hipLaunchKernelGGL(k_blind_rotate1w2, dim3(B), dim3(64 * kWaves), 0, s, in, n0, bk, tv,
+                       tv_stride, out, int(sample_extract), B);
     return hipGetLastError();
 }
 

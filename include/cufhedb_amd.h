@@ -357,9 +357,10 @@ int fhe_digit_testvectors(int op, int digits, int digit_bits, uint64_t threshold
  * fhe_tune_set read and restore the table (e.g. from a per-device cache). */
 enum fhe_tune_knob {
     FHE_TUNE_IKS21_TILE = 0, /* ciphertexts per workgroup: 8, 16, 32, 64      */
-    FHE_TUNE_PBS1_WAVES = 1, /* waves per ciphertext of the FP64 lvl1 blind
-                                rotation: 1, or 2 (small batches: each
-                                ciphertext's CMUX on two SIMDs); untuned: 2
+    FHE_TUNE_PBS1_WAVES = 1, /* waves per polynomial of the FP64 lvl1 blind
+                                rotation: 1 (one wave per ciphertext), or 2
+                                (small batches: the digit rows of a CMUX side
+                                by side on one compute unit); untuned: 2
                                 below 512 ciphertexts */
     FHE_TUNE_IKS_SPLIT = 2,  /* workgroups per ciphertext of the lvl1 -> lvl0
                                 key switch (kind 10; 1, 2, 4, 8: the digit
