@@ -358,6 +358,13 @@ __device__ __forceinline__ void fft512_inv2(cd a[8], cd b[8], cd *lds, int lane,
 
 constexpr int kLaneTile = 320;  // double2 per wave tile of lanes64_fwd / lanes64_inv
 
+// A twiddle base whose powers are formed again at each use: the compiler
+// would keep them in registers (8 a base), which kernels with four waves per
+// SIMD do not have.
+struct FreshBase {
+    cd b;
+};
+
 // v[q] *= base^q (CONJ: conj(base)^q), q = 1..3
 template <bool CONJ>
 __device__ __forceinline__ void twiddle4(cd v[4], cd base)
@@ -367,6 +374,13 @@ __device__ __forceinline__ void twiddle4(cd v[4], cd base)
     v[1] = CONJ ? cmulc(v[1], base) : cmul(v[1], base);
     v[2] = CONJ ? cmulc(v[2], b2) : cmul(v[2], b2);
     v[3] = CONJ ? cmulc(v[3], b3) : cmul(v[3], b3);
+}
+
+template <bool CONJ>
+__device__ __forceinline__ void twiddle4(cd v[4], FreshBase t)
+{
+    asm volatile("" : "+v"(t.b.x), "+v"(t.b.y));
+    twiddle4<CONJ>(v, t.b);
 }
 
 // Exchange of one 32-bit word between two registers across lane groups:
@@ -427,8 +441,8 @@ __device__ __forceinline__ void transpose_reg_lane_hi_lds(cd v[4], cd *tile, int
 // t64 = W64^(lane & 15), t16 = W16^(lane & 3).  Input: register r, lane L
 // holds x_r[L]; output: register q, lane l holds X_r[m] for r = l >> 4,
 // m = ((l >> 2) & 3) + 4 (l & 3) + 16 q.
-template <bool PERM>
-__device__ __forceinline__ void lanes64_fwd(cd v[4], cd *tile, int l, cd t64, cd t16)
+template <bool PERM, class Tw>
+__device__ __forceinline__ void lanes64_fwd(cd v[4], cd *tile, int l, Tw t64, Tw t16)
 {
     // T1: (lane L, reg m1) -> lane (L0 = l & 15, m1 = l >> 4), reg L1
     if constexpr (PERM)
@@ -456,8 +470,8 @@ __device__ __forceinline__ void lanes64_fwd(cd v[4], cd *tile, int l, cd t64, cd
     dft4<1>(v[0], v[1], v[2], v[3]);
 }
 
-template <bool PERM>
-__device__ __forceinline__ void lanes64_inv(cd v[4], cd *tile, int l, cd t64, cd t16)
+template <bool PERM, class Tw>
+__device__ __forceinline__ void lanes64_inv(cd v[4], cd *tile, int l, Tw t64, Tw t16)
 {
     dft4<-1>(v[0], v[1], v[2], v[3]);
 #pragma unroll

@@ -68,6 +68,12 @@ __device__ __forceinline__ TwQ make_twq(int lane, int wave)
     return t;
 }
 
+// the same, the passes' twiddle powers not kept
+struct TwQFresh {
+    cd beta, rho;
+    FreshBase t256, t64, t16;
+};
+
 // c_p = exp(i pi p / 8)
 __device__ __forceinline__ cd cq(int p)
 {
@@ -76,37 +82,74 @@ __device__ __forceinline__ cd cq(int p)
 }
 
 // Forward: v[p] = z[lane + 64 wave + 256 p] in, Z[4 m' + wave] (layout above)
-// out.  xch: the workgroup's 4 x 256 double2 exchange area, which aliases the
-// four wave tiles (tiles = xch + wave * kTileQ).
-template <bool PERM = false>
-__device__ __forceinline__ void fft1024q_fwd(cd v[4], cd *xch, int lane, int wave, const TwQ &tw)
+// out, in two parts around the exchange between the polynomial's four waves.
+// xch: their four tiles (tile k at xch + k kTileQ); part A computes the wave's
+// words of the four sequences, the caller exchanges them (sequence k at the
+// start of tile k), part C goes on in the wave's own tile, which no other
+// wave touches until the next exchange.
+template <class Tw>
+__device__ __forceinline__ void fft1024q_fwd_a(cd v[4], const Tw &tw)
 {
     v[1] = cmul(v[1], cq(1));
     v[2] = cmul(v[2], cq(2));
     v[3] = cmul(v[3], cq(3));
     dft4<1>(v[0], v[1], v[2], v[3]);
-    {
-        cd g = tw.beta;
+    cd g = tw.beta;
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            v[k] = cmul(v[k], g);
-            if (k < 3) g = cmul(g, tw.rho);
-        }
+    for (int k = 0; k < 4; k++) {
+        v[k] = cmul(v[k], g);
+        if (k < 3) g = cmul(g, tw.rho);
     }
-    const int n0 = lane + 64 * wave;
-    // the exchange area overlaps the wave tiles: every wave has left its tile
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 4; k++) xch[k * kTileQ + n0] = v[k];
-    __syncthreads();
-    // wave k's sequence sits at the start of wave k's own tile, so the wave
-    // may go on into its tile without waiting for the others' reads
-#pragma unroll
-    for (int j = 0; j < 4; j++) v[j] = xch[wave * kTileQ + lane + 64 * j];
+}
+
+template <bool PERM, class Tw>
+__device__ __forceinline__ void fft1024q_fwd_c(cd v[4], cd *tile, int lane, const Tw &tw)
+{
     // step C: radix-4 over the registers (stride 64), twiddle W256^{L m1}
     dft4<1>(v[0], v[1], v[2], v[3]);
     twiddle4<false>(v, tw.t256);
-    lanes64_fwd<PERM>(v, xch + wave * kTileQ, lane, tw.t64, tw.t16);
+    lanes64_fwd<PERM>(v, tile, lane, tw.t64, tw.t16);
+}
+
+template <bool PERM = false>
+__device__ __forceinline__ void fft1024q_fwd(cd v[4], cd *xch, int lane, int wave, const TwQ &tw)
+{
+    fft1024q_fwd_a(v, tw);
+    // the exchange area overlaps the wave tiles: every wave has left its tile
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; k++) xch[k * kTileQ + lane + 64 * wave] = v[k];
+    __syncthreads();
+    cd *tile = xch + wave * kTileQ;
+#pragma unroll
+    for (int j = 0; j < 4; j++) v[j] = tile[lane + 64 * j];
+    fft1024q_fwd_c<PERM>(v, tile, lane, tw);
+}
+
+// The inverse in two parts around its exchange (words lane + 64 j of the
+// wave's sequence after part A, the wave's words of the four sequences before
+// part C).
+template <bool PERM, class Tw>
+__device__ __forceinline__ void fft1024q_inv_a(cd v[4], cd *tile, int lane, const Tw &tw)
+{
+    lanes64_inv<PERM>(v, tile, lane, tw.t64, tw.t16);
+    twiddle4<true>(v, tw.t256);
+    dft4<-1>(v[0], v[1], v[2], v[3]);
+}
+
+template <class Tw>
+__device__ __forceinline__ void fft1024q_inv_c(cd v[4], const Tw &tw)
+{
+    cd g = tw.beta;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        v[k] = cmulc(v[k], g);
+        if (k < 3) g = cmul(g, tw.rho);
+    }
+    dft4<-1>(v[0], v[1], v[2], v[3]);
+    v[1] = cmulc(v[1], cq(1));
+    v[2] = cmulc(v[2], cq(2));
+    v[3] = cmulc(v[3], cq(3));
 }
 
 // TAIL_SYNC: wait for every wave's exchange reads before returning (the
@@ -116,31 +159,18 @@ __device__ __forceinline__ void fft1024q_fwd(cd v[4], cd *xch, int lane, int wav
 template <bool PERM = false, bool TAIL_SYNC = true>
 __device__ __forceinline__ void fft1024q_inv(cd v[4], cd *xch, int lane, int wave, const TwQ &tw)
 {
-    lanes64_inv<PERM>(v, xch + wave * kTileQ, lane, tw.t64, tw.t16);
-    twiddle4<true>(v, tw.t256);
-    dft4<-1>(v[0], v[1], v[2], v[3]);
+    cd *tile = xch + wave * kTileQ;
+    fft1024q_inv_a<PERM>(v, tile, lane, tw);
     // the wave writes its own tile, which no other wave reads or writes
     // between the last barrier (a forward exchange's second, or the previous
     // inverse's tail) and the reads below: no barrier before the write
 #pragma unroll
-    for (int j = 0; j < 4; j++) xch[wave * kTileQ + lane + 64 * j] = v[j];
+    for (int j = 0; j < 4; j++) tile[lane + 64 * j] = v[j];
     __syncthreads();
-    const int n0 = lane + 64 * wave;
 #pragma unroll
-    for (int k = 0; k < 4; k++) v[k] = xch[k * kTileQ + n0];
+    for (int k = 0; k < 4; k++) v[k] = xch[k * kTileQ + lane + 64 * wave];
     if (TAIL_SYNC) __syncthreads();
-    {
-        cd g = tw.beta;
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            v[k] = cmulc(v[k], g);
-            if (k < 3) g = cmul(g, tw.rho);
-        }
-    }
-    dft4<-1>(v[0], v[1], v[2], v[3]);
-    v[1] = cmulc(v[1], cq(1));
-    v[2] = cmulc(v[2], cq(2));
-    v[3] = cmulc(v[3], cq(3));
+    fft1024q_inv_c(v, tw);
 }
 
 // natural frequency of (wave, lane, register q) in the output layout
@@ -217,14 +247,13 @@ constexpr int kQRow = 4 * 4 * 64;  // double2 per (i, row, column): [wave][q][la
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_blind_rotate2q(
     const uint32_t *__restrict__ in, int n0, const cd *__restrict__ bk,
     const cd *__restrict__ rot, const uint64_t *__restrict__ tv, int tv_stride, int tv_period,
-    uint64_t *__restrict__ out, int sample_extract, int B)
+    uint64_t *__restrict__ out, int sample_extract)
 {
     __shared__ uint64_t acc[2 * N2q];
     __shared__ cd xch[4 * kTileQ];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ct = blockIdx.x;
-    if (ct >= B) return;
     const uint32_t *c0 = in + size_t(ct) * (n0 + 1);
     const uint64_t *tvp = tv + size_t(tv_period > 0 ? ct % tv_period : ct) * tv_stride;
     const TwQ tw = make_twq(lane, wave);
@@ -329,6 +358,205 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     }
 }
 
+constexpr int kRowWavesQ = 16;  // four quarters of each of a column's four digit rows
+
+// LDS of one small-batch blind rotation (156 KB of the CU's 160).  The
+// accumulator (prepared as above) is kept as high and low words: three of
+// the four digits read only the high ones, one word a lane.
+struct alignas(16) Br2sLds {
+    cd row[kRowWavesQ][kTileQ];  // row waves' tiles, then their row's spectrum
+    cd col[8][kTileQ];           // product sums, then the inverse's tiles (column, quarter)
+    uint32_t hi[2][N2q], lo[2][N2q];
+    uint32_t step[kMaxN0 + 1];
+};
+static_assert(64 * kRowWavesQ >= kMaxN0, "one thread per step");
+
+// Small batches: a compute unit per ciphertext, its 16 waves transforming the
+// four digit rows of a column at once (wave = row d, quarter w).  A CMUX step
+// takes column 0's rows, then column 1's:
+//   rows:     digits and transform of the row, spectrum left in the tiles;
+//   products: wave (quarter, register) sums the column's rows into both
+//             output columns for its 64 points, rows in ascending order, with
+//             the key words loaded since the previous products;
+// then X^abar - 1 is applied to the sums, and eight waves (column, quarter)
+// run the inverses and update the accumulator.  Each value is computed by the
+// operations of k_blind_rotate2q in the same order.
+//
+// Bound by LDS: about 12,900 of a step's 18,000 cycles move its words (writes
+// at 74-80 bytes a clock), and the transforms' VALU work fills the SIMDs to a
+// similar share.  One MI355X, n0 = 672, up to 256 ciphertexts: 5.2-5.4 ms
+// against 7.9 for k_blind_rotate2q, which has one wave per SIMD there.  Words
+// that stay with their wave in an exchange (one of four) skip LDS; the key
+// loads are spread over the row phases, because issued together they hold the
+// waves up at the L1's 64 bytes a clock (6.3 ms); the powers of the passes'
+// twiddles are formed at each use, since read from LDS tables they cost its
+// time (6.5 ms) and kept in registers they spill.
+__global__ __launch_bounds__(64 * kRowWavesQ) void k_blind_rotate2s(
+    const uint32_t *__restrict__ in, int n0, const cd *__restrict__ bk,
+    const cd *__restrict__ rot, const uint64_t *__restrict__ tv, int tv_stride, int tv_period,
+    uint64_t *__restrict__ out, int sample_extract)
+{
+    __shared__ Br2sLds lds;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ct = blockIdx.x;
+    const uint32_t *c0 = in + size_t(ct) * (n0 + 1);
+    const uint64_t *tvp = tv + size_t(tv_period > 0 ? ct % tv_period : ct) * tv_stride;
+    const int w = wave & 3, d = wave >> 2;  // as a row wave: quarter, digit
+    const TwQ t = make_twq(lane, w);
+    const TwQFresh tw{t.beta, t.rho, {t.t256}, {t.t64}, {t.t16}};
+
+    const uint32_t bbar = 2u * N2q - (c0[n0] >> (32 - 1 - Lvl2::nbit));
+    auto put = [&](int c, int n, uint64_t u) {
+        lds.hi[c][n] = uint32_t(u >> 32);
+        lds.lo[c][n] = uint32_t(u);
+    };
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const int n = tid + 1024 * k;
+        const uint32_t idx = (uint32_t(n) - bbar) & (2u * N2q - 1);
+        const uint64_t v = tvp[idx & (N2q - 1)];
+        put(0, n, prep2q(0));
+        put(1, n, prep2q((idx & N2q) ? 0ull - v : v));
+    }
+    // the steps with a rotation to do (a-bar = 0 is skipped), in order, as
+    // i << 12 | a-bar
+    constexpr uint32_t kRound = 1u << (32 - 2 - Lvl2::nbit);
+    {
+        const uint32_t abar = tid < n0 ? (c0[tid] + kRound) >> (32 - 1 - Lvl2::nbit) : 0u;
+        const uint64_t some = __ballot(abar != 0);
+        int *rank = reinterpret_cast<int *>(lds.row);
+        if (lane == 0) rank[wave] = __popcll(some);
+        __syncthreads();
+        int at = 0, all = 0;
+        for (int k = 0; k < kRowWavesQ; k++) {
+            if (k == wave) at = all;
+            all += rank[k];
+        }
+        if (abar) lds.step[at + __popcll(some & ((1ull << lane) - 1))] = uint32_t(tid) << 12 | abar;
+        if (tid == 0) lds.step[all] = 0;
+    }
+    // as a product wave: quarter w, register d; the exponent of its points is
+    // e0 + 1024 d (k_blind_rotate2q)
+    const uint32_t e0 = 4u * uint32_t(q_freq(w, lane, 0)) + 1u;
+    cd key[2 * Lvl2::l];
+    auto load_key = [&](uint32_t step, int c, int r0, int r1) {
+        const cd *k = bk + (size_t(step >> 12) * Lvl2::rows + c * Lvl2::l) * 2 * kQRow + w * 256 +
+                      d * 64 + lane;
+#pragma unroll
+        for (int r = r0; r < r1; r++) key[r] = k[r * kQRow];
+    };
+    // word by word: as a whole, a conditional load becomes a select of
+    // pointers and v moves to scratch
+    auto get = [](cd &x, const cd *p) {
+        x.x = p->x;
+        x.y = p->y;
+    };
+    __syncthreads();
+    uint32_t step = __builtin_amdgcn_readfirstlane(lds.step[0]);
+
+    for (int k = 1; step; k++) {
+        const uint32_t abar = step & 0xfffu;
+        cd fd[2] = {{0.0, 0.0}, {0.0, 0.0}}, base{};
+#pragma unroll 1
+        for (int c = 0; c < 2; c++) {
+            // compared where they are used: hoisted, the comparisons would be
+            // kept as lane masks and selected
+            int ws = w, ds = d;
+            asm volatile("" : "+s"(ws), "+s"(ds));
+            cd v[4];
+            auto digits = [&](auto word, int sh) {
+#pragma unroll
+                for (int p = 0; p < 4; p++) {
+                    const int n = lane + 64 * w + 256 * p;
+                    v[p] = cd{double(int32_t(__builtin_amdgcn_sbfe(int32_t(word(n)), sh, Lvl2::Bgbit))),
+                              double(int32_t(__builtin_amdgcn_sbfe(int32_t(word(n + 1024)), sh, Lvl2::Bgbit)))};
+                }
+            };
+            if (d < Lvl2::l - 1)
+                digits([&](int n) { return lds.hi[c][n]; }, 32 - Lvl2::Bgbit * (d + 1));
+            else  // the last digit: bits 28 to 36
+                digits([&](int n) { return __builtin_amdgcn_alignbit(lds.hi[c][n], lds.lo[c][n], 28); }, 0);
+            load_key(step, c, 0, 2);
+            fft1024q_fwd_a(v, tw);
+            if (c == 1) __syncthreads();  // column 0's products have read the tiles
+            // the wave keeps its own words of its own sequence (v[w]), and below
+            // its own row's points of its products (v[d])
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (j != ws) lds.row[4 * d + j][lane + 64 * w] = v[j];
+            load_key(step, c, 2, 4);
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (j != ws) get(v[j], lds.row[wave] + lane + 64 * j);
+            load_key(step, c, 4, 6);
+            fft1024q_fwd_c<true>(v, lds.row[wave], lane, tw);
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (q != ds) lds.row[wave][q * 64 + lane] = v[q];
+            load_key(step, c, 6, 8);
+            if (c == 1) base = rot[(abar * e0) & (2u * N2q - 1)];
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < Lvl2::l; r++) {
+                cd s = v[r];
+                if (r != ds) get(s, lds.row[4 * r + w] + d * 64 + lane);
+                cmac(fd[0], s, key[2 * r]);
+                cmac(fd[1], s, key[2 * r + 1]);
+            }
+        }
+        {
+            cd g = mul_ipow2q(base, abar * uint32_t(d));
+            g.x -= 1.0;
+            lds.col[w][d * 64 + lane] = cmul(fd[0], g);
+            lds.col[4 + w][d * 64 + lane] = cmul(fd[1], g);
+        }
+        const uint32_t ahead = lds.step[k];
+        __syncthreads();
+        cd v[4];
+        cd *tile = lds.col[wave & 7];
+        if (wave >= 8) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[q] = tile[q * 64 + lane];
+            wave_lds_sync();
+            fft1024q_inv_a<true>(v, tile, lane, tw);
+#pragma unroll
+            for (int j = 0; j < 4; j++) tile[lane + 64 * j] = v[j];
+        }
+        step = __builtin_amdgcn_readfirstlane(ahead);
+        __syncthreads();
+        if (wave >= 8) {
+            const int c = (wave >> 2) & 1;
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = lds.col[4 * c + j][lane + 64 * w];
+            fft1024q_inv_c(v, tw);
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int n = lane + 64 * w + 256 * (j >> 1) + 1024 * (j & 1);
+                const uint64_t u = uint64_t(lds.hi[c][n]) << 32 | lds.lo[c][n];
+                put(c, n, prep2q(unprep2q(u) + trunc_torus64q(j & 1 ? v[j >> 1].y : v[j >> 1].x)));
+            }
+        }
+        __syncthreads();
+    }
+
+    auto word = [&](int c, int n) {
+        return unprep2q(uint64_t(lds.hi[c][n]) << 32 | lds.lo[c][n]);
+    };
+    if (sample_extract) {
+        uint64_t *o = out + size_t(ct) * (N2q + 1);
+        for (int n = tid; n < N2q; n += 1024) o[n] = n == 0 ? word(0, 0) : 0ull - word(0, N2q - n);
+        if (tid == 0) o[N2q] = word(1, 0);
+    } else {
+        uint64_t *o = out + size_t(ct) * 2 * N2q;
+        for (int n = tid; n < N2q; n += 1024) {
+            o[n] = word(0, n);
+            o[N2q + n] = word(1, n);
+        }
+    }
+}
+
 // integer torus polynomial -> key layout [wave][q][lane], scaled by 1/1024
 __global__ __launch_bounds__(256) void k_poly_to_devfd2q(const uint64_t *__restrict__ poly,
                                                           cd *__restrict__ fd, int npoly)
@@ -383,6 +611,14 @@ __global__ __launch_bounds__(256) void k_ifft2q(const uint64_t *__restrict__ pol
 
 }  // namespace
 
+// Up to one ciphertext per compute unit k_blind_rotate2s is faster (one
+// MI355X, n0 = 672: 5.4 against 7.9 ms); beyond, its second round costs as
+// much as k_blind_rotate2q's two or three ciphertexts per unit (10.8 against
+// 10.9 ms at 300, 16.2 against 12.8 at 768), and at the end of a large batch
+// it would replace a part round that costs k_blind_rotate2q only 4.3 ms
+// (4096 against 3840 ciphertexts).
+constexpr int kSmall2q = 256;
+
 size_t bk2q_device_elems(int n0) { return size_t(n0) * Lvl2::rows * 2 * kQRow; }
 
 hipError_t launch_bk2q_from_int(const uint64_t *bk_int, cd *bk_dev, int n0, hipStream_t s)
@@ -397,8 +633,12 @@ hipError_t launch_blind_rotate2q(const uint32_t *in, int n0, const cd *bk, const
                                  bool sample_extract, int B, hipStream_t s, int tv_period)
 {
     if (B <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_blind_rotate2q, dim3(B), dim3(256), 0, s, in, n0, bk, rot, tv, tv_stride,
-                       tv_period, out, int(sample_extract), B);
+    if (B <= kSmall2q)
+        hipLaunchKernelGGL(k_blind_rotate2s, dim3(B), dim3(64 * kRowWavesQ), 0, s, in, n0, bk, rot,
+                           tv, tv_stride, tv_period, out, int(sample_extract));
+    else
+        hipLaunchKernelGGL(k_blind_rotate2q, dim3(B), dim3(256), 0, s, in, n0, bk, rot, tv,
+                           tv_stride, tv_period, out, int(sample_extract));
     return hipGetLastError();
 }
 
