@@ -431,7 +431,8 @@ class Context:
 
     def autotune(self, batches=(64, 256, 1024, 4096, 16384), knob=None):
         """Time every candidate of `knob` (TUNE_IKS21_TILE: ciphertexts per
-        workgroup of the lvl2 -> lvl1 key switch, needs KSK 21;
+        workgroup of the lvl2 -> lvl1 key switch, 8 and 16 standing for 128,
+        32 for 256 and 64 for 512, needs KSK 21;
         TUNE_PBS1_WAVES: waves per ciphertext of the lvl1 blind rotation,
         needs BK lvl01; TUNE_IKS_SPLIT / TUNE_IKS20_SPLIT: workgroups per
         ciphertext of the lvl1 -> lvl0 / lvl2 -> lvl0 key switch, needs KSK

@@ -71,6 +71,40 @@ int prepare_pbs1(fhe_ctx *ctx, hipStream_t s)
     return FHE_OK;
 }
 
+int ksk_target(fhe_ctx *ctx, int kind, uint32_t **dst)
+{
+    uint32_t *&slot = ctx->ksk[ksk_slot(kind)];
+    *dst = kind == 21 ? nullptr : slot;
+    if (*dst) return FHE_OK;
+    const size_t bytes = (fhe_ksk_words(&ctx->p, kind) + kKskPadWords) * sizeof(uint32_t);
+    HIP_TRY(hipMalloc(dst, bytes), "KSK allocation");
+    if (kind != 21) slot = *dst;
+    return FHE_OK;
+}
+
+int ksk_commit(fhe_ctx *ctx, int kind, uint32_t *dst)
+{
+    if (kind != 21) return FHE_OK;
+    uint32_t *&slot = ctx->ksk[ksk_slot(kind)];
+    uint32_t *to = slot;
+    hipError_t e = to ? hipSuccess : hipMalloc(&to, ksk21_bytes());
+    if (e == hipSuccess) e = launch_ksk21_layout(dst, to, ctx->stream);
+    const hipError_t es = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) e = es;
+    ksk_drop(kind, dst);
+    if (e == hipSuccess)
+        slot = to;
+    else if (to && !slot)
+        (void)hipFree(to);
+    HIP_TRY(e, "KSK 21 layout");
+    return FHE_OK;
+}
+
+void ksk_drop(int kind, uint32_t *dst)
+{
+    if (kind == 21 && dst) (void)hipFree(dst);
+}
+
 // lvl1 blind rotation (+ sample extraction) with the context's variant
 int launch_pbs1(fhe_ctx *ctx, const uint32_t *in, const uint32_t *tv, int tv_stride,
                 uint32_t *out, bool se, int B, hipStream_t s)
@@ -258,9 +292,14 @@ int fhe_load_ksk(fhe_ctx *ctx, int kind, const uint32_t *ksk_host)
     FHE_CHECK_ARG(slot >= 0, "fhe_load_ksk: kind must be 10, 20 or 21 (got %d)", kind);
     HIP_TRY(hipSetDevice(ctx->device), "hipSetDevice");
     const size_t bytes = fhe_ksk_words(&ctx->p, kind) * sizeof(uint32_t);
-    if (int rc = alloc_ksk(ctx, kind)) return rc;
-    HIP_TRY(hipMemcpy(ctx->ksk[slot], ksk_host, bytes, hipMemcpyHostToDevice), "KSK upload");
-    return FHE_OK;
+    uint32_t *dst = nullptr;
+    if (int rc = ksk_target(ctx, kind, &dst)) return rc;
+    const hipError_t e = hipMemcpy(dst, ksk_host, bytes, hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        ksk_drop(kind, dst);
+        return hip_fail(e, "KSK upload");
+    }
+    return ksk_commit(ctx, kind, dst);
 }
 
 int fhe_bk_loaded(const fhe_ctx *ctx, int level)

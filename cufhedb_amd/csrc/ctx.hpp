@@ -112,19 +112,20 @@ inline int grow(uint32_t *&buf, size_t &cap, size_t words)
     return FHE_OK;
 }
 
-// Device key-switching keys are allocated with kKskPadWords spare words at
-// the end: the whole-row key-switch kernel reads every row in 64-word chunks
-// and may run up to 63 words past the end of the last row (those words are
-// discarded).
+// Device keys of kinds 10 and 20 are allocated with kKskPadWords spare words
+// at the end: the whole-row key-switch kernel reads every row in 64-word
+// chunks and may run up to 63 words past the end of the last row (those words
+// are discarded).
 constexpr size_t kKskPadWords = 64;
-inline int alloc_ksk(fhe_ctx *ctx, int kind)
-{
-    const int slot = ksk_slot(kind);
-    if (ctx->ksk[slot]) return FHE_OK;
-    const size_t bytes = (fhe_ksk_words(&ctx->p, kind) + kKskPadWords) * sizeof(uint32_t);
-    HIP_TRY(hipMalloc(&ctx->ksk[slot], bytes), "KSK allocation");
-    return FHE_OK;
-}
+
+// A key-switching key's way onto the device (capi.hip): ksk_target gives the
+// buffer that receives it in the reference layout (the context's slot; for
+// kind 21 a temporary one), ksk_commit puts it into service (kind 21: into the
+// slot in the matrix product's layout) and ksk_drop gives a temporary buffer
+// back without that.
+int ksk_target(fhe_ctx *ctx, int kind, uint32_t **dst);
+int ksk_commit(fhe_ctx *ctx, int kind, uint32_t *dst);
+void ksk_drop(int kind, uint32_t *dst);
 
 // tuned value of `knob` for a batch of B, or `dflt` if the knob is untuned
 inline int tuned(const fhe_ctx *ctx, int knob, int B, int dflt)
@@ -136,16 +137,16 @@ inline int tuned(const fhe_ctx *ctx, int knob, int B, int dflt)
     return v;
 }
 
-// workgroup shape of a key switch of B ciphertexts.  Kind 21: ciphertexts
-// per workgroup; untuned 8 below 512 ciphertexts, 16 below 2048, else 32
-// (one MI355X: 32 ciphertexts 1.9 / 2.7 / 9.2 ms with tiles 8 / 16 / 32,
-// 2048 ciphertexts 19.1 / 17.3 / 13.6 ms).  Kinds 10 and 20: workgroups per
+// workgroup shape of a key switch of B ciphertexts.  Kind 21: 512, 256 or 128
+// ciphertexts per workgroup (launch_iks21; one MI355X, 64 / 32 / 16: 100
+// ciphertexts 0.20 / 0.15 / 0.15 ms, 256 0.19 / 0.15 / 0.22, 300 0.20 / 0.24 /
+// 0.32, 4096 1.25 / 1.69 / 2.65).  Kinds 10 and 20: workgroups per
 // ciphertext over the digit positions; untuned 8 (one MI355X, n0 = 672, split
 // 1 / 8: kind 10 16 ciphertexts 0.13 / 0.02 ms, 16384 ciphertexts 15.1 /
 // 13.5 ms; kind 20 16384 ciphertexts 31.0 / 28.6 ms).
 inline int iks_tile(const fhe_ctx *ctx, int kind, int B)
 {
-    if (kind == 21) return tuned(ctx, FHE_TUNE_IKS21_TILE, B, B < 256 ? 8 : B < 512 ? 16 : 64);
+    if (kind == 21) return tuned(ctx, FHE_TUNE_IKS21_TILE, B, B <= 128 ? 16 : B <= 256 ? 32 : 64);
     return tuned(ctx, kind == 10 ? FHE_TUNE_IKS_SPLIT : FHE_TUNE_IKS20_SPLIT, B, 8);
 }
 

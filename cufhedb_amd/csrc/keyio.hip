@@ -319,10 +319,14 @@ int stream_to_device(fhe_ctx *ctx, File &f, void *dst_dev, uint64_t bytes, int e
 
 int load_ksk_stream(fhe_ctx *ctx, File &f, int ks_kind, uint64_t bytes)
 {
-    const int slot = ksk_slot(ks_kind);
     HIP_TRY(hipSetDevice(ctx->device), "hipSetDevice");
-    if (int rc = alloc_ksk(ctx, ks_kind)) return rc;
-    return stream_to_device(ctx, f, ctx->ksk[slot], bytes, 4);
+    uint32_t *dst = nullptr;
+    if (int rc = ksk_target(ctx, ks_kind, &dst)) return rc;
+    if (int rc = stream_to_device(ctx, f, dst, bytes, 4)) {
+        ksk_drop(ks_kind, dst);
+        return rc;
+    }
+    return ksk_commit(ctx, ks_kind, dst);
 }
 
 int load_bk_from_file(fhe_ctx *ctx, File &f, int level, int format, uint64_t bytes, int elem)

@@ -86,11 +86,16 @@ hipError_t launch_sample_extract2(const uint64_t *trlwe, uint64_t *tlwe, int ind
 
 // ---- identity key switching and small element-wise ops, iks.hip ---------
 // kind 10: uint32 domain (dn = 1024), kind 20/21: uint64 domain (dn = 2048)
-// tile: kind 21, ciphertexts per workgroup (8, 16, 32; 0 = 32); kinds 10
-// and 20, workgroups per ciphertext over the digit positions (1, 2, 4, 8;
-// 0 = 1)
+// tile: kind 21 (ksk in launch_ksk21_layout's layout), ciphertexts per
+// workgroup: 512 (64), 256 (32) or 128 (else); kinds 10 and 20, workgroups per ciphertext over the digit positions (1, 2, 4, 8; 0 = 1)
 hipError_t launch_iks(int kind, const void *in, const uint32_t *ksk, uint32_t *out, int tn, int B,
                       hipStream_t s, int tile = 0);
+// lvl2 -> lvl1 on the matrix cores (iks21.hip): the key's own layout, built
+// from the reference layout, and the switch
+size_t ksk21_bytes();
+hipError_t launch_ksk21_layout(const uint32_t *ksk, uint32_t *dst, hipStream_t s);
+hipError_t launch_iks21(const uint64_t *in, const uint32_t *key, uint32_t *out, int B, int tile,
+                        hipStream_t s);
 // out = sa*a + sb*b (+ offset on the body word), lvl1 TLWEs of 1025 words
 hipError_t launch_tlwe1_lincomb(const uint32_t *a, const uint32_t *b, int sa, int sb,
                                 uint32_t offset, uint32_t *out, int B, hipStream_t s);

@@ -344,19 +344,18 @@ int fhe_digit_testvectors(int op, int digits, int digit_bits, uint64_t threshold
 /* ---- tile autotuning ---------------------------------------------------- */
 /* No reference counterpart (the reference launches one ciphertext per call).
  * FHE_TUNE_IKS21_TILE: ciphertexts per workgroup of the lvl2 -> lvl1 key
- * switch: 8, 16 or 32 with one output column per lane (more read each key
- * row once for more ciphertexts, fewer give small batches more workgroups),
- * or 64 with one ciphertext per lane (key rows staged in LDS; the fastest
- * form from about 512 ciphertexts up).  fhe_autotune
+ * switch: 128 (8 and 16), 256 (32) or 512 (64); more read each key block
+ * once for more ciphertexts, fewer leave less of a small batch's workgroups
+ * empty.  fhe_autotune
  * times every candidate on the context's KSK 21 at the n ascending batch
  * sizes and keeps the fastest per size (a batch then uses the entry of the
- * largest size <= it; untuned: 8 below 256 ciphertexts, 16 below 512,
+ * largest size <= it; untuned: 16 up to 128 ciphertexts, 32 up to 256,
  * else 64); choice (n, may be NULL) receives the picks, ms (n x the
  * knob's candidate count, in candidate order, may be NULL) the mean
  * times.  All candidates compute identical results.  fhe_tune_get /
  * fhe_tune_set read and restore the table (e.g. from a per-device cache). */
 enum fhe_tune_knob {
-    FHE_TUNE_IKS21_TILE = 0, /* ciphertexts per workgroup: 8, 16, 32, 64      */
+    FHE_TUNE_IKS21_TILE = 0, /* 8, 16: 128 ciphertexts per workgroup, 32: 256, 64: 512 */
     FHE_TUNE_PBS1_WAVES = 1, /* waves per polynomial of the FP64 lvl1 blind
                                 rotation: 1 (one wave per ciphertext), or 2
                                 (small batches: the digit rows of a CMUX side
