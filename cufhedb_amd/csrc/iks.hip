@@ -7,10 +7,11 @@
 //                       if a_ij != 0: res -= ksk[i][j][a_ij - 1]
 // The reference runs this on the host CPU before every bootstrap
 // (src/cuHEDB/gatebootstrap_gpu.cuh:42,59,...).  Here a batch is one launch
-// of k_iks_rows (kinds 10 and 20, basebit 10), which reads every selected key
-// row whole from the reference's own layout [dn][t][2^basebit - 1][tn + 1],
-// one workgroup per ciphertext, or the matrix product of iks21.hip (kind 21,
-// basebit 3).
+// from the reference's own key layout [dn][t][2^basebit - 1][tn + 1] for kinds
+// 10 and 20 (basebit 10), where k_iks_rows reads every selected row whole, one
+// workgroup per ciphertext, and k_iks_gather, for large batches, stages the
+// rows of a position in LDS for 4096 ciphertexts; kind 21 (basebit 3) is the
+// matrix product of iks21.hip.
 #include "launch.hpp"
 #include "params.hpp"
 
@@ -116,6 +117,173 @@ void launch_iks_rows(const TD *in, const uint32_t *ksk, uint32_t *out, int tn, i
     }
     hipLaunchKernelGGL((k_iks_rows<TD, DN, T, BB, NCH>), dim3(B, split), dim3(256), 0, s, in, ksk,
                        out, tn, B);
+}
+
+// Gather form of the same switch for batches that select every key row
+// several times: a workgroup of 1024 threads takes four ciphertexts per thread
+// (1024 apart) on a slice of 16 output columns and a range of digit positions.
+// A position's 1023 rows on the slice (64 KB, behind a zero row for digit 0)
+// are staged in LDS, two buffers, the next position's words in flight in
+// registers, and every lane adds the row that its digit selects: the key is
+// read once per 4096 ciphertexts instead of once per ciphertext.  A row's four
+// 16-byte chunks are rotated by its number (chunk k at k ^ (r >> 2)) so that
+// the lanes' random rows meet all the banks.
+//
+// Bound by the key's way into the compute units: 64 KB a position in 64-byte
+// pieces of 2692-byte rows, 4.0 TB/s over the chip (without it 8192
+// ciphertexts take 2.3 of their 3.8 ms).  One MI355X, n0 = 672, against a
+// workgroup per ciphertext: kind 10 2.0 against 2.5 ms at 3000 ciphertexts,
+// 3.8 against 6.7 at 8192, 6.5 against 13.5 at 16384; kind 20 3.8 against 5.3,
+// 7.3 against 14.3, 14.0 against 28.7.  Not kept: two ciphertexts per thread
+// (4.6 at 8192), one word per load (4.2), each lane adding its own columns to
+// the output (a line per lane: 9.1).
+constexpr int kGatherCols = 16, kGatherPer = 4;
+// from these batches on (kind 10 / 20): one round of the key costs the gather
+// form 1.4-1.6 / 2.8-3.2 ms whatever the batch, k_iks_rows 0.82 / 1.75 us a
+// ciphertext (2200: 1.86 against 1.82 ms, 2400: 1.92 against 1.99; kind 20,
+// 1500: 3.27 against 2.64, 2048: 3.44 against 3.59)
+constexpr int kGatherFrom10 = 2400, kGatherFrom20 = 2048;
+
+template <class TD, int DN, int T, int BB>
+__global__ __launch_bounds__(1024) void k_iks_gather(const TD *__restrict__ in,
+                                                     const uint32_t *__restrict__ ksk,
+                                                     uint32_t *__restrict__ out, int tn, int B,
+                                                     int slices, int tiles, int per)
+{
+    constexpr int W = int(sizeof(TD) * 8);
+    constexpr uint32_t mask = (1u << BB) - 1;
+    constexpr int kRowsLds = 1 << BB;               // candidate rows, row 0 zero
+    constexpr int kWords = 16 / int(sizeof(TD));    // mask words loaded at a time
+    constexpr int kStep = kWords * T;               // positions between loads
+    static_assert(kRowsLds == 1024 && T == 2, "one 16-byte chunk in four per thread and row");
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    __shared__ __align__(16) u32x4 buf[2][kRowsLds * 4];
+    const int tid = threadIdx.x;
+    // workgroups go to the eight XCDs in turn: an XCD's take the tiles and
+    // slices of the same positions, which share the key rows' cache lines
+    const int xcd = blockIdx.x & 7, loc = blockIdx.x >> 3;
+    const int tile = loc % tiles, c0 = loc / tiles % slices * kGatherCols;
+    const int split = xcd + 8 * (loc / tiles / slices);
+    const int e0 = split * per, e1 = min(e0 + per, DN * T);
+    if (e0 >= e1) return;
+    const size_t row = size_t(tn) + 1;
+
+    // chunk c of LDS row r: threads take rows tid / 4 + 256 k
+    const int c = tid & 3;
+    u32x4 v[4];
+    const uint32_t row4 = uint32_t(row) * 4u;
+    const uint32_t voff = uint32_t(tid >> 2) * row4 + 16u * c;  // of LDS row tid / 4 + 1
+    auto fetch = [&](int e) {
+        const char *base = reinterpret_cast<const char *>(ksk + size_t(e) * mask * row + c0);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            // key row tid / 4 + 256 k - 1; its place before the first is not stored
+            const uint32_t o = k ? voff + (256u * k - 1u) * row4 : voff >= row4 ? voff - row4 : voff;
+            __builtin_memcpy(&v[k], base + o, 16);
+        }
+    };
+    auto store = [&](int b) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int r = (tid >> 2) + 256 * k;
+            if (r) buf[b][4 * r + (c ^ ((r >> 2) & 3))] = v[k];
+        }
+    };
+    if (tid < 8) buf[tid >> 2][tid & 3] = u32x4{0, 0, 0, 0};
+
+    // the next kWords mask words of this thread's ciphertexts (the digits are
+    // in the upper halves of 64-bit ones)
+    const int b0 = tile * 1024 * kGatherPer + tid;
+    u32x4 raw[kGatherPer];
+    uint32_t acc[kGatherPer][kGatherCols];
+#pragma unroll
+    for (int n = 0; n < kGatherPer; n++)
+#pragma unroll
+        for (int k = 0; k < kGatherCols; k++) acc[n][k] = 0;
+
+    fetch(e0);
+    for (int e = e0; e < e1; e += kStep) {
+#pragma unroll
+        for (int n = 0; n < kGatherPer; n++)
+            __builtin_memcpy(&raw[n], in + size_t(min(b0 + 1024 * n, B - 1)) * (DN + 1) + e / T, 16);
+#pragma unroll 1
+        for (int w = 0; w < kWords; w++) {
+#pragma unroll
+            for (int u = 0; u < T; u++) {
+                const int p = e + T * w + u;
+                store(u);
+                if (p + 1 < e1) fetch(p + 1);
+                __syncthreads();
+                const char *rows = reinterpret_cast<const char *>(buf[u]);
+#pragma unroll
+                for (int n = 0; n < kGatherPer; n++) {
+                    // a wave's 64 ciphertexts are neighbours: none of them
+                    // left, nothing to add
+                    if (__builtin_amdgcn_readfirstlane(b0 + 1024 * n) >= B) break;
+                    const uint32_t x = raw[n][W == 32 ? 0 : 1] + (1u << (31 - BB * T));
+                    const uint32_t d = x >> (32 - (u + 1) * BB) & mask;
+                    const uint32_t at = d << 6 | (d << 2 & 0x30u);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const u32x4 y = *reinterpret_cast<const u32x4 *>(rows + (at ^ uint32_t(16 * k)));
+#pragma unroll
+                        for (int q = 0; q < 4; q++) acc[n][4 * k + q] += y[q];
+                    }
+                    // one ciphertext's reads at a time, for their registers
+#pragma unroll
+                    for (int k = 0; k < kGatherCols; k++) asm volatile("" : "+v"(acc[n][k]));
+                }
+            }
+#pragma unroll
+            for (int n = 0; n < kGatherPer; n++)
+                raw[n] = W == 32 ? __builtin_shufflevector(raw[n], raw[n], 1, 2, 3, 3)
+                                 : __builtin_shufflevector(raw[n], raw[n], 2, 3, 3, 3);
+        }
+    }
+    // 1024 ciphertexts at a time through LDS, so that the additions go out as
+    // 16 adjacent words
+    constexpr int kPad = kGatherCols + 1;
+    uint32_t *flat = reinterpret_cast<uint32_t *>(buf);
+    const int col = c0 + (tid & (kGatherCols - 1));
+#pragma unroll
+    for (int n = 0; n < kGatherPer; n++) {
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kGatherCols; q++) flat[tid * kPad + q] = acc[n][q];
+        __syncthreads();
+        const int first = tile * 1024 * kGatherPer + 1024 * n;
+        for (int r = tid / kGatherCols; r < 1024 && first + r < B; r += 1024 / kGatherCols) {
+            const size_t b = size_t(first + r);
+            uint32_t x = 0u - flat[r * kPad + col - c0];
+            if (split == 0 && col == tn) {
+                const TD y = in[b * (DN + 1) + DN];
+                x += W == 32 ? uint32_t(y) : uint32_t((y + (TD(1) << (W - 33))) >> (W - 32));
+            }
+            if (col <= tn) atomicAdd(out + b * row + col, x);
+        }
+    }
+}
+
+template <class TD, int DN, int T, int BB>
+void launch_iks_gather(const TD *in, const uint32_t *ksk, uint32_t *out, int tn, int B, hipStream_t s)
+{
+    const int slices = (tn + 1 + kGatherCols - 1) / kGatherCols;
+    const int tiles = (B + 1024 * kGatherPer - 1) / (1024 * kGatherPer);
+    constexpr int kStep = 16 / int(sizeof(TD)) * T;
+    auto range = [](int k) { return (DN * T / kStep + k - 1) / k * kStep; };
+    // splits of the positions, eight at a time (one an XCD), so that the
+    // workgroups fill the 256 compute units (one each), against about three
+    // positions' worth of start and end per workgroup
+    int split = 8;
+    long best = 0;
+    for (int k = 8; k <= 64; k += 8) {
+        const long cost = (long(slices) * tiles * k + 255) / 256 * (range(k) + 3);
+        if (k == 8 || cost < best) best = cost, split = k;
+    }
+    const size_t n = size_t(B) * (tn + 1);
+    hipLaunchKernelGGL(k_fill_zero32, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, out, n);
+    hipLaunchKernelGGL((k_iks_gather<TD, DN, T, BB>), dim3(unsigned(slices * tiles * split)),
+                       dim3(1024), 0, s, in, ksk, out, tn, B, slices, tiles, range(split));
 }
 
 __global__ void k_tlwe1_lincomb(const uint32_t *__restrict__ a, const uint32_t *__restrict__ b,
@@ -288,14 +456,20 @@ hipError_t launch_iks(int kind, const void *in, const uint32_t *ksk, uint32_t *o
     switch (kind) {
     case 10:
     case 20: {
-        // `tile` = workgroups per ciphertext over the digit positions
+        // `tile` = workgroups per ciphertext over the digit positions; with 8
+        // of them the gather form takes over where it is faster
         const int split = tile == 2 || tile == 4 || tile == 8 ? tile : 1;
-        if (kind == 10)
-            launch_iks_rows<uint32_t, Lvl1::N, KS10::t, KS10::basebit>(
-                static_cast<const uint32_t *>(in), ksk, out, tn, B, split, s);
+        const bool gather = split == 8 && B >= (kind == 10 ? kGatherFrom10 : kGatherFrom20);
+        const auto *x1 = static_cast<const uint32_t *>(in);
+        const auto *x2 = static_cast<const uint64_t *>(in);
+        if (kind == 10 && gather)
+            launch_iks_gather<uint32_t, Lvl1::N, KS10::t, KS10::basebit>(x1, ksk, out, tn, B, s);
+        else if (kind == 10)
+            launch_iks_rows<uint32_t, Lvl1::N, KS10::t, KS10::basebit>(x1, ksk, out, tn, B, split, s);
+        else if (gather)
+            launch_iks_gather<uint64_t, Lvl2::N, KS20::t, KS20::basebit>(x2, ksk, out, tn, B, s);
         else
-            launch_iks_rows<uint64_t, Lvl2::N, KS20::t, KS20::basebit>(
-                static_cast<const uint64_t *>(in), ksk, out, tn, B, split, s);
+            launch_iks_rows<uint64_t, Lvl2::N, KS20::t, KS20::basebit>(x2, ksk, out, tn, B, split, s);
         break;
     }
     case 21:

@@ -87,7 +87,9 @@ hipError_t launch_sample_extract2(const uint64_t *trlwe, uint64_t *tlwe, int ind
 // ---- identity key switching and small element-wise ops, iks.hip ---------
 // kind 10: uint32 domain (dn = 1024), kind 20/21: uint64 domain (dn = 2048)
 // tile: kind 21 (ksk in launch_ksk21_layout's layout), ciphertexts per
-// workgroup: 512 (64), 256 (32) or 128 (else); kinds 10 and 20, workgroups per ciphertext over the digit positions (1, 2, 4, 8; 0 = 1)
+// workgroup: 512 (64), 256 (32) or 128 (else); kinds 10 and 20, workgroups per
+// ciphertext over the digit positions (1, 2, 4, 8; 0 = 1; with 8, large
+// batches take k_iks_gather)
 hipError_t launch_iks(int kind, const void *in, const uint32_t *ksk, uint32_t *out, int tn, int B,
                       hipStream_t s, int tile = 0);
 // lvl2 -> lvl1 on the matrix cores (iks21.hip): the key's own layout, built
