@@ -73,18 +73,50 @@ int prepare_pbs1(fhe_ctx *ctx, hipStream_t s)
 
 int ksk_target(fhe_ctx *ctx, int kind, uint32_t **dst)
 {
+    const size_t words = fhe_ksk_words(&ctx->p, kind);
+    if (kind == 21) {
+        *dst = nullptr;
+        HIP_TRY(hipMalloc(dst, words * sizeof(uint32_t)), "KSK allocation");
+        return FHE_OK;
+    }
     uint32_t *&slot = ctx->ksk[ksk_slot(kind)];
-    *dst = kind == 21 ? nullptr : slot;
-    if (*dst) return FHE_OK;
-    const size_t bytes = (fhe_ksk_words(&ctx->p, kind) + kKskPadWords) * sizeof(uint32_t);
-    HIP_TRY(hipMalloc(dst, bytes), "KSK allocation");
-    if (kind != 21) slot = *dst;
+    const int tn = int(ctx->p.n0);
+    const size_t spread = words / (tn + 1) * ksk_row_words(tn);
+    if (!slot)
+        HIP_TRY(hipMalloc(&slot, (spread + kKskPadWords) * sizeof(uint32_t)), "KSK allocation");
+    *dst = slot + (spread - words);
     return FHE_OK;
 }
 
+namespace {
+
+// rows of kinds 10 and 20 from the end of the slot's buffer to their places
+int spread_ksk(fhe_ctx *ctx, int kind)
+{
+    const int tn = int(ctx->p.n0);
+    if (ksk_row_words(tn) == tn + 1) return FHE_OK;
+    const size_t rows = fhe_ksk_words(&ctx->p, kind) / (tn + 1), tmp_rows = size_t(1) << 14;
+    uint32_t *tmp = nullptr;
+    hipError_t e = hipMalloc(&tmp, tmp_rows * (tn + 1) * sizeof(uint32_t));
+    if (e == hipSuccess)
+        e = launch_ksk_spread(ctx->ksk[ksk_slot(kind)], tn, rows, tmp, tmp_rows, ctx->stream);
+    const hipError_t es = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) e = es;
+    (void)hipFree(tmp);
+    if (e != hipSuccess) {
+        // half moved: not a key any more
+        (void)hipFree(ctx->ksk[ksk_slot(kind)]);
+        ctx->ksk[ksk_slot(kind)] = nullptr;
+    }
+    HIP_TRY(e, "KSK layout");
+    return FHE_OK;
+}
+
+}  // namespace
+
 int ksk_commit(fhe_ctx *ctx, int kind, uint32_t *dst)
 {
-    if (kind != 21) return FHE_OK;
+    if (kind != 21) return spread_ksk(ctx, kind);
     uint32_t *&slot = ctx->ksk[ksk_slot(kind)];
     uint32_t *to = slot;
     hipError_t e = to ? hipSuccess : hipMalloc(&to, ksk21_bytes());

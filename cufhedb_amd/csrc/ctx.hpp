@@ -114,15 +114,15 @@ inline int grow(uint32_t *&buf, size_t &cap, size_t words)
 
 // Device keys of kinds 10 and 20 are allocated with kKskPadWords spare words
 // at the end: the whole-row key-switch kernel reads every row in 64-word
-// chunks and may run up to 63 words past the end of the last row (those words
-// are discarded).
+// chunks and may run past the end of the last row (those words are
+// discarded).
 constexpr size_t kKskPadWords = 64;
 
 // A key-switching key's way onto the device (capi.hip): ksk_target gives the
-// buffer that receives it in the reference layout (the context's slot; for
-// kind 21 a temporary one), ksk_commit puts it into service (kind 21: into the
-// slot in the matrix product's layout) and ksk_drop gives a temporary buffer
-// back without that.
+// buffer that receives it in the reference layout (the end of the context's
+// slot; for kind 21 a temporary one), ksk_commit puts it into service (its
+// rows spread to whole lines; kind 21: into the slot in the matrix product's
+// layout) and ksk_drop gives a temporary buffer back without that.
 int ksk_target(fhe_ctx *ctx, int kind, uint32_t **dst);
 int ksk_commit(fhe_ctx *ctx, int kind, uint32_t *dst);
 void ksk_drop(int kind, uint32_t *dst);

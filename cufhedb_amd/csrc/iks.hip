@@ -8,10 +8,10 @@
 // The reference runs this on the host CPU before every bootstrap
 // (src/cuHEDB/gatebootstrap_gpu.cuh:42,59,...).  Here a batch is one launch
 // from the reference's own key layout [dn][t][2^basebit - 1][tn + 1] for kinds
-// 10 and 20 (basebit 10), where k_iks_rows reads every selected row whole, one
-// workgroup per ciphertext, and k_iks_gather, for large batches, stages the
-// rows of a position in LDS for 4096 ciphertexts; kind 21 (basebit 3) is the
-// matrix product of iks21.hip.
+// 10 and 20 (basebit 10), rows at whole 128-byte lines (ksk_row_words), where
+// k_iks_rows reads every selected row whole, one workgroup per ciphertext, and
+// k_iks_gather, for large batches, stages the rows of a position in LDS for
+// 4096 ciphertexts; kind 21 (basebit 3) is the matrix product of iks21.hip.
 #include "launch.hpp"
 #include "params.hpp"
 
@@ -28,7 +28,8 @@ namespace {
 // per wave; the four waves' partial sums meet in LDS.  The loop body has no
 // branch: a zero digit reads a valid row and discards it, and lanes past the
 // last column read up to 63 words beyond the row (the device key carries
-// kKskPadWords spare words) into sums that are never written.
+// kKskPadWords spare words) into sums that are never written.  (Rows at whole
+// lines: 1.63 ms for 2000 ciphertexts of kind 10, 1.66 when packed.)
 template <class TD, int DN, int T, int BB, int NCH>
 __global__ __launch_bounds__(256) void k_iks_rows(const TD *__restrict__ in,
                                                   const uint32_t *__restrict__ ksk,
@@ -55,7 +56,7 @@ __global__ __launch_bounds__(256) void k_iks_rows(const TD *__restrict__ in,
     __syncthreads();
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const size_t row = size_t(tn) + 1;
+    const size_t row = size_t(tn) + 1, stride = size_t(ksk_row_words(tn));
     uint32_t acc[NCH];
 #pragma unroll
     for (int j = 0; j < NCH; j++) acc[j] = 0;
@@ -63,8 +64,8 @@ __global__ __launch_bounds__(256) void k_iks_rows(const TD *__restrict__ in,
         const uint32_t d0 = __builtin_amdgcn_readfirstlane(uint32_t(dig[e]));
         const uint32_t d1 = __builtin_amdgcn_readfirstlane(uint32_t(dig[e + 4]));
         const uint32_t keep0 = d0 ? 0xffffffffu : 0u, keep1 = d1 ? 0xffffffffu : 0u;
-        const uint32_t *k0 = ksk + (size_t(e) * nd + (d0 ? d0 - 1 : 0)) * row + lane;
-        const uint32_t *k1 = ksk + (size_t(e + 4) * nd + (d1 ? d1 - 1 : 0)) * row + lane;
+        const uint32_t *k0 = ksk + (size_t(e) * nd + (d0 ? d0 - 1 : 0)) * stride + lane;
+        const uint32_t *k1 = ksk + (size_t(e + 4) * nd + (d1 ? d1 - 1 : 0)) * stride + lane;
         uint32_t v0[NCH], v1[NCH];
 #pragma unroll
         for (int j = 0; j < NCH; j++) v0[j] = k0[64 * j];
@@ -120,29 +121,33 @@ void launch_iks_rows(const TD *in, const uint32_t *ksk, uint32_t *out, int tn, i
 }
 
 // Gather form of the same switch for batches that select every key row
-// several times: a workgroup of 1024 threads takes four ciphertexts per thread
-// (1024 apart) on a slice of 16 output columns and a range of digit positions.
-// A position's 1023 rows on the slice (64 KB, behind a zero row for digit 0)
-// are staged in LDS, two buffers, the next position's words in flight in
-// registers, and every lane adds the row that its digit selects: the key is
-// read once per 4096 ciphertexts instead of once per ciphertext.  A row's four
-// 16-byte chunks are rotated by its number (chunk k at k ^ (r >> 2)) so that
-// the lanes' random rows meet all the banks.
+// several times: a workgroup of 1024 threads takes 4096 ciphertexts on a slice
+// of 16 output columns and a range of digit positions.  A position's 1023 rows
+// on the slice (64 KB, behind a zero row for digit 0) are staged in LDS, two
+// buffers, the next position's words in flight in registers; a quad of lanes
+// holds the slice's sums of 16 ciphertexts, four columns a lane, and adds the
+// rows that their digits select: the key is read once per 4096 ciphertexts
+// instead of once per ciphertext.  A quad's read is a row's 64 bytes, so the
+// four quads that LDS serves in a cycle meet in its four bank groups; with a
+// whole row per lane 16 lanes met in 16.  The digits come as byte offsets
+// through LDS, each formed by one thread of the workgroup.
 //
 // Bound by the key's way into the compute units: 64 KB a position in 64-byte
-// pieces of 2692-byte rows, 4.0 TB/s over the chip (without it 8192
-// ciphertexts take 2.3 of their 3.8 ms).  One MI355X, n0 = 672, against a
-// workgroup per ciphertext: kind 10 2.0 against 2.5 ms at 3000 ciphertexts,
-// 3.8 against 6.7 at 8192, 6.5 against 13.5 at 16384; kind 20 3.8 against 5.3,
-// 7.3 against 14.3, 14.0 against 28.7.  Not kept: two ciphertexts per thread
-// (4.6 at 8192), one word per load (4.2), each lane adding its own columns to
-// the output (a line per lane: 9.1).
-constexpr int kGatherCols = 16, kGatherPer = 4;
+// pieces of rows, one line each (without it 8192 ciphertexts take 2.0 of their
+// 3.0 ms; rows packed without regard to lines, 2692 bytes apart: 3.4).  One
+// MI355X, n0 = 672, against a row per lane on packed rows: kind 10 1.7 against
+// 1.9 ms at 2400 ciphertexts, 2.1 against 2.5 at 4096, 3.0 against 3.8 at
+// 8192, 5.0 against 6.6 at 16384; kind 20 3.0 against 3.5 at 2048, 5.9 against
+// 7.4 at 8192.  Not kept: mask words loaded two at a time for their registers
+// (the words' lines are read again: 3.2 at 8192), slices stored one after the
+// other (2.7 at 8192, but 64-byte pieces double k_iks_rows' time).
+constexpr int kGatherCols = 16, kGatherPer = 16;  // columns a workgroup, ciphertexts a quad
+constexpr int kGatherTile = 256 * kGatherPer;     // ciphertexts a workgroup
 // from these batches on (kind 10 / 20): one round of the key costs the gather
-// form 1.4-1.6 / 2.8-3.2 ms whatever the batch, k_iks_rows 0.82 / 1.75 us a
-// ciphertext (2200: 1.86 against 1.82 ms, 2400: 1.92 against 1.99; kind 20,
-// 1500: 3.27 against 2.64, 2048: 3.44 against 3.59)
-constexpr int kGatherFrom10 = 2400, kGatherFrom20 = 2048;
+// form 1.5-2.1 / 2.8-3.6 ms whatever the batch, k_iks_rows 0.81 / 1.7 us a
+// ciphertext (1800: 1.57 against 1.45 ms, 2000: 1.62 against 1.63; kind 20,
+// 1600: 2.86 against 2.73, 1800: 2.91 against 3.07)
+constexpr int kGatherFrom10 = 2000, kGatherFrom20 = 1700;
 
 template <class TD, int DN, int T, int BB>
 __global__ __launch_bounds__(1024) void k_iks_gather(const TD *__restrict__ in,
@@ -157,7 +162,11 @@ __global__ __launch_bounds__(1024) void k_iks_gather(const TD *__restrict__ in,
     constexpr int kStep = kWords * T;               // positions between loads
     static_assert(kRowsLds == 1024 && T == 2, "one 16-byte chunk in four per thread and row");
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    __shared__ __align__(16) u32x4 buf[2][kRowsLds * 4];
+    struct alignas(16) Lds {
+        u32x4 row[2][kRowsLds * 4];
+        uint16_t at[2][256][kGatherPer];  // byte offset of the row that a ciphertext selects
+    };
+    __shared__ Lds lds;
     const int tid = threadIdx.x;
     // workgroups go to the eight XCDs in turn: an XCD's take the tiles and
     // slices of the same positions, which share the key rows' cache lines
@@ -167,91 +176,111 @@ __global__ __launch_bounds__(1024) void k_iks_gather(const TD *__restrict__ in,
     const int e0 = split * per, e1 = min(e0 + per, DN * T);
     if (e0 >= e1) return;
     const size_t row = size_t(tn) + 1;
+    const uint32_t stride = uint32_t(ksk_row_words(tn));
 
     // chunk c of LDS row r: threads take rows tid / 4 + 256 k
     const int c = tid & 3;
     u32x4 v[4];
-    const uint32_t row4 = uint32_t(row) * 4u;
+    const uint32_t row4 = stride * 4u;
     const uint32_t voff = uint32_t(tid >> 2) * row4 + 16u * c;  // of LDS row tid / 4 + 1
     auto fetch = [&](int e) {
-        const char *base = reinterpret_cast<const char *>(ksk + size_t(e) * mask * row + c0);
+        const char *base = reinterpret_cast<const char *>(ksk + size_t(e) * mask * stride + c0);
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             // key row tid / 4 + 256 k - 1; its place before the first is not stored
             const uint32_t o = k ? voff + (256u * k - 1u) * row4 : voff >= row4 ? voff - row4 : voff;
-            __builtin_memcpy(&v[k], base + o, 16);
+            v[k] = *reinterpret_cast<const u32x4 *>(base + o);
         }
     };
     auto store = [&](int b) {
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int r = (tid >> 2) + 256 * k;
-            if (r) buf[b][4 * r + (c ^ ((r >> 2) & 3))] = v[k];
-        }
+        for (int k = 0; k < 4; k++)
+            if (k || tid >= 4) lds.row[b][tid + 1024 * k] = v[k];
     };
-    if (tid < 8) buf[tid >> 2][tid & 3] = u32x4{0, 0, 0, 0};
+    if (tid < 8) lds.row[tid >> 2][tid & 3] = u32x4{0, 0, 0, 0};
 
-    // the next kWords mask words of this thread's ciphertexts (the digits are
-    // in the upper halves of 64-bit ones)
-    const int b0 = tile * 1024 * kGatherPer + tid;
-    u32x4 raw[kGatherPer];
-    uint32_t acc[kGatherPer][kGatherCols];
+    // ciphertext of quad g = tid / 4 and sum n: b0 + 256 n + g.  This thread
+    // provides the digits of quad `dg`, sums 4 dn to 4 dn + 3: raw holds their
+    // next kWords mask words (the digits are in the upper halves of 64-bit ones)
+    const int b0 = tile * kGatherTile, g = tid >> 2, dg = tid & 255, dn = tid >> 8;
+    u32x4 raw[kGatherPer / 4];
+    uint32_t acc[kGatherPer][4];
 #pragma unroll
     for (int n = 0; n < kGatherPer; n++)
 #pragma unroll
-        for (int k = 0; k < kGatherCols; k++) acc[n][k] = 0;
+        for (int k = 0; k < 4; k++) acc[n][k] = 0;
+
+    auto load_words = [&](int e) {
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+            const size_t b = size_t(min(b0 + 256 * (4 * dn + m) + dg, B - 1));
+            __builtin_memcpy(&raw[m], in + b * (DN + 1) + e / T, 16);
+        }
+    };
 
     fetch(e0);
+    load_words(e0);
     for (int e = e0; e < e1; e += kStep) {
-#pragma unroll
-        for (int n = 0; n < kGatherPer; n++)
-            __builtin_memcpy(&raw[n], in + size_t(min(b0 + 1024 * n, B - 1)) * (DN + 1) + e / T, 16);
 #pragma unroll 1
         for (int w = 0; w < kWords; w++) {
 #pragma unroll
             for (int u = 0; u < T; u++) {
                 const int p = e + T * w + u;
                 store(u);
+                uint32_t x[4];
+#pragma unroll
+                for (int m = 0; m < 4; m++) {
+                    const uint32_t d = (raw[m][W == 32 ? 0 : 1] + (1u << (31 - BB * T))) >> (32 - (u + 1) * BB);
+                    x[m] = (d & mask) << 6;
+                }
+                *reinterpret_cast<uint64_t *>(&lds.at[u][dg][4 * dn]) =
+                    uint64_t(x[2] | x[3] << 16) << 32 | (x[0] | x[1] << 16);
+                if (u == T - 1) {
+#pragma unroll
+                    for (int m = 0; m < 4; m++)
+                        raw[m] = W == 32 ? __builtin_shufflevector(raw[m], raw[m], 1, 2, 3, 3)
+                                         : __builtin_shufflevector(raw[m], raw[m], 2, 3, 3, 3);
+                    if (w == kWords - 1 && p + 1 < e1) load_words(p + 1);
+                }
                 if (p + 1 < e1) fetch(p + 1);
                 __syncthreads();
-                const char *rows = reinterpret_cast<const char *>(buf[u]);
+                const char *rows = reinterpret_cast<const char *>(lds.row[u]) + 16 * c;
+                const u32x4 *at = reinterpret_cast<const u32x4 *>(lds.at[u][g]);
 #pragma unroll
-                for (int n = 0; n < kGatherPer; n++) {
-                    // a wave's 64 ciphertexts are neighbours: none of them
-                    // left, nothing to add
-                    if (__builtin_amdgcn_readfirstlane(b0 + 1024 * n) >= B) break;
-                    const uint32_t x = raw[n][W == 32 ? 0 : 1] + (1u << (31 - BB * T));
-                    const uint32_t d = x >> (32 - (u + 1) * BB) & mask;
-                    const uint32_t at = d << 6 | (d << 2 & 0x30u);
+                for (int h = 0; h < kGatherPer / 8; h++) {
+                    const u32x4 o = at[h];
 #pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        const u32x4 y = *reinterpret_cast<const u32x4 *>(rows + (at ^ uint32_t(16 * k)));
+                    for (int j = 0; j < 8; j++) {
+                        const int n = 8 * h + j;
+                        const uint32_t a = j & 1 ? o[j >> 1] >> 16 : o[j >> 1] & 0xffffu;
+                        const u32x4 y = *reinterpret_cast<const u32x4 *>(rows + a);
 #pragma unroll
-                        for (int q = 0; q < 4; q++) acc[n][4 * k + q] += y[q];
+                        for (int q = 0; q < 4; q++) acc[n][q] += y[q];
+                        // four rows' reads at a time, for their registers
+                        if (j & 4 ? j == 7 : j == 3)
+#pragma unroll
+                            for (int k = n - 3; k <= n; k++)
+#pragma unroll
+                                for (int q = 0; q < 4; q++) asm volatile("" : "+v"(acc[k][q]));
                     }
-                    // one ciphertext's reads at a time, for their registers
-#pragma unroll
-                    for (int k = 0; k < kGatherCols; k++) asm volatile("" : "+v"(acc[n][k]));
                 }
             }
-#pragma unroll
-            for (int n = 0; n < kGatherPer; n++)
-                raw[n] = W == 32 ? __builtin_shufflevector(raw[n], raw[n], 1, 2, 3, 3)
-                                 : __builtin_shufflevector(raw[n], raw[n], 2, 3, 3, 3);
         }
     }
     // 1024 ciphertexts at a time through LDS, so that the additions go out as
     // 16 adjacent words
     constexpr int kPad = kGatherCols + 1;
-    uint32_t *flat = reinterpret_cast<uint32_t *>(buf);
+    uint32_t *flat = reinterpret_cast<uint32_t *>(lds.row);
     const int col = c0 + (tid & (kGatherCols - 1));
 #pragma unroll
-    for (int n = 0; n < kGatherPer; n++) {
+    for (int n = 0; n < kGatherPer; n += 4) {
         __syncthreads();
 #pragma unroll
-        for (int q = 0; q < kGatherCols; q++) flat[tid * kPad + q] = acc[n][q];
+        for (int m = 0; m < 4; m++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) flat[(256 * m + g) * kPad + 4 * c + q] = acc[n + m][q];
         __syncthreads();
-        const int first = tile * 1024 * kGatherPer + 1024 * n;
+        const int first = b0 + 256 * n;
         for (int r = tid / kGatherCols; r < 1024 && first + r < B; r += 1024 / kGatherCols) {
             const size_t b = size_t(first + r);
             uint32_t x = 0u - flat[r * kPad + col - c0];
@@ -264,11 +293,24 @@ __global__ __launch_bounds__(1024) void k_iks_gather(const TD *__restrict__ in,
     }
 }
 
+// rows first .. first + count - 1, packed in src, to their places in the key;
+// the words between them are zeroed
+__global__ __launch_bounds__(256) void k_ksk_spread(const uint32_t *__restrict__ src,
+                                                    uint32_t *__restrict__ key, int row, int stride,
+                                                    size_t count)
+{
+    const size_t gid = size_t(blockIdx.x) * 256 + threadIdx.x;
+    if (gid >= count * stride) return;
+    const size_t r = gid / stride;
+    const int k = int(gid % stride);
+    key[gid] = k < row ? src[r * row + k] : 0u;
+}
+
 template <class TD, int DN, int T, int BB>
 void launch_iks_gather(const TD *in, const uint32_t *ksk, uint32_t *out, int tn, int B, hipStream_t s)
 {
     const int slices = (tn + 1 + kGatherCols - 1) / kGatherCols;
-    const int tiles = (B + 1024 * kGatherPer - 1) / (1024 * kGatherPer);
+    const int tiles = (B + kGatherTile - 1) / kGatherTile;
     constexpr int kStep = 16 / int(sizeof(TD)) * T;
     auto range = [](int k) { return (DN * T / kStep + k - 1) / k * kStep; };
     // splits of the positions, eight at a time (one an XCD), so that the
@@ -448,6 +490,25 @@ hipError_t launch_tv_ide(T *tv, uint32_t scale_bits, int N, hipStream_t s)
 }
 template hipError_t launch_tv_ide<uint32_t>(uint32_t *, uint32_t, int, hipStream_t);
 template hipError_t launch_tv_ide<uint64_t>(uint64_t *, uint32_t, int, hipStream_t);
+
+hipError_t launch_ksk_spread(uint32_t *key, int tn, size_t rows, uint32_t *tmp, size_t tmp_rows,
+                             hipStream_t s)
+{
+    const size_t row = size_t(tn) + 1, stride = size_t(ksk_row_words(tn));
+    // the packed rows start rows * (stride - row) words into the buffer, so a
+    // row's place ends before the next packed row starts: in ascending order,
+    // a part at a time through tmp, no row is overwritten before it is read
+    const uint32_t *packed = key + rows * (stride - row);
+    for (size_t r = 0; r < rows; r += tmp_rows) {
+        const size_t n = rows - r < tmp_rows ? rows - r : tmp_rows;
+        const hipError_t e = hipMemcpyAsync(tmp, packed + r * row, n * row * sizeof(uint32_t),
+                                            hipMemcpyDeviceToDevice, s);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(k_ksk_spread, dim3(unsigned((n * stride + 255) / 256)), dim3(256), 0, s,
+                           tmp, key + r * stride, int(row), int(stride), n);
+    }
+    return hipGetLastError();
+}
 
 hipError_t launch_iks(int kind, const void *in, const uint32_t *ksk, uint32_t *out, int tn, int B,
                       hipStream_t s, int tile)

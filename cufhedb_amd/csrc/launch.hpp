@@ -90,6 +90,13 @@ hipError_t launch_sample_extract2(const uint64_t *trlwe, uint64_t *tlwe, int ind
 // workgroup: 512 (64), 256 (32) or 128 (else); kinds 10 and 20, workgroups per
 // ciphertext over the digit positions (1, 2, 4, 8; 0 = 1; with 8, large
 // batches take k_iks_gather)
+// ksk of kinds 10 and 20: the reference layout [dn][t][2^basebit - 1][tn + 1]
+// with rows ksk_row_words(tn) words apart, at whole 128-byte lines
+constexpr int ksk_row_words(int tn) { return (tn + 1 + 31) & ~31; }
+// spreads `rows` rows of tn + 1 words, packed at the end of the key's buffer,
+// to that distance in place; tmp: room for tmp_rows >= 1 packed rows
+hipError_t launch_ksk_spread(uint32_t *key, int tn, size_t rows, uint32_t *tmp, size_t tmp_rows,
+                             hipStream_t s);
 hipError_t launch_iks(int kind, const void *in, const uint32_t *ksk, uint32_t *out, int tn, int B,
                       hipStream_t s, int tile = 0);
 // lvl2 -> lvl1 on the matrix cores (iks21.hip): the key's own layout, built
