@@ -61,12 +61,84 @@ __device__ __forceinline__ cd c8w(int p)
     return p == 1 ? cd{c1, s1} : p == 2 ? cd{kR2, kR2} : cd{s1, c1};
 }
 
+// The exchanges of the transforms.  A wave keeps the words of its own two
+// sequences and trades the others with the other half, two words a lane each
+// way: put_* before the caller's barrier, get_* behind it on the tile that the
+// other half wrote.  Forward (seqs), from the four sequences' words at the
+// wave's n0 to its sequence s at n0 of half h in register 2 s + h; inverse
+// (parts), back.  The empty asm keeps the two branches apart: merged, a load
+// becomes one into a selected register and v moves to scratch.  (Whole
+// exchanges through LDS: 2.39 against 2.35 ms at one ciphertext, 4.9 against
+// 4.75 at 300.)
+__device__ __forceinline__ void put_seqs(const cd v[4], cd *tile, int lane, int half)
+{
+    if (half == 0) {
+        asm volatile("; half 0: in");
+        tile[lane] = v[2];
+        tile[64 + lane] = v[3];
+        asm volatile("; half 0: out");
+    } else {
+        asm volatile("; half 1: in");
+        tile[lane] = v[0];
+        tile[64 + lane] = v[1];
+        asm volatile("; half 1: out");
+    }
+}
+
+__device__ __forceinline__ void get_seqs(cd v[4], const cd *tile, int lane, int half)
+{
+    if (half == 0) {
+        asm volatile("; half 0: in");
+        v[2] = v[1];
+        v[1] = tile[lane];
+        v[3] = tile[64 + lane];
+        asm volatile("; half 0: out");
+    } else {
+        asm volatile("; half 1: in");
+        v[1] = v[2];
+        v[0] = tile[lane];
+        v[2] = tile[64 + lane];
+        asm volatile("; half 1: out");
+    }
+}
+
+__device__ __forceinline__ void put_parts(const cd v[4], cd *tile, int lane, int half)
+{
+    if (half == 0) {
+        asm volatile("; half 0: in");
+        tile[lane] = v[1];
+        tile[64 + lane] = v[3];
+        asm volatile("; half 0: out");
+    } else {
+        asm volatile("; half 1: in");
+        tile[lane] = v[0];
+        tile[64 + lane] = v[2];
+        asm volatile("; half 1: out");
+    }
+}
+
+__device__ __forceinline__ void get_parts(cd v[4], const cd *tile, int lane, int half)
+{
+    if (half == 0) {
+        asm volatile("; half 0: in");
+        v[1] = v[2];
+        v[2] = tile[lane];
+        v[3] = tile[64 + lane];
+        asm volatile("; half 0: out");
+    } else {
+        asm volatile("; half 1: in");
+        v[2] = v[1];
+        v[0] = tile[lane];
+        v[1] = tile[64 + lane];
+        asm volatile("; half 1: out");
+    }
+}
+
 // The forward transform of one wave's half, in two parts around the exchange
-// between the two halves (the caller's barrier).  pair: the two halves' tiles
-// (2 x kLaneTile double2); part A puts sequence k of half v = k >> 1 at the
-// start of v's tile, part C goes on in the half's own tile, which no other
-// wave touches until the next exchange.
-__device__ __forceinline__ void fft512w_fwd_a(cd v[4], cd *pair, int lane, int half, const TwW &tw)
+// between the two halves (the caller's barrier): part A puts the other half's
+// words into its tile (theirs), part C goes on in the half's own tile, which
+// no other wave touches until the next exchange.
+__device__ __forceinline__ void fft512w_fwd_a(cd v[4], cd *theirs, int lane, int half, const TwW &tw)
 {
     v[1] = cmul(v[1], c8w(1));
     v[2] = cmul(v[2], c8w(2));
@@ -80,15 +152,13 @@ __device__ __forceinline__ void fft512w_fwd_a(cd v[4], cd *pair, int lane, int h
             if (k < 3) g = cmul(g, tw.rho);
         }
     }
-    const int n0 = lane + 64 * half;
-#pragma unroll
-    for (int k = 0; k < 4; k++) pair[(k >> 1) * kLaneTile + (k & 1) * 128 + n0] = v[k];
+    put_seqs(v, theirs, lane, half);
 }
 
-__device__ __forceinline__ void fft512w_fwd_c(cd v[4], cd *tile, int lane, const TwW &tw)
+__device__ __forceinline__ void fft512w_fwd_c(cd v[4], cd *tile, int lane, int half, const TwW &tw)
 {
-#pragma unroll
-    for (int j = 0; j < 4; j++) v[j] = tile[(j >> 1) * 128 + lane + 64 * (j & 1)];
+    get_seqs(v, tile, lane, half);
+    wave_lds_sync();
 #pragma unroll
     for (int s = 0; s < 2; s++) {
         const cd a = v[2 * s], b = v[2 * s + 1];
@@ -99,9 +169,9 @@ __device__ __forceinline__ void fft512w_fwd_c(cd v[4], cd *tile, int lane, const
 }
 
 // The inverse (unnormalised: returns 512 z), frequency layout in, time layout
-// out, in two parts around the exchange: part A ends with the wave's words in
-// its own tile, part C reads both halves' tiles.
-__device__ __forceinline__ void fft512w_inv_a(cd v[4], cd *tile, int lane, const TwW &tw)
+// out, in two parts around the exchange: part A ends with the other half's
+// words in the wave's own tile, part C reads the other half's tile.
+__device__ __forceinline__ void fft512w_inv_a(cd v[4], cd *tile, int lane, int half, const TwW &tw)
 {
     lanes64_inv<true>(v, tile, lane, tw.t64, tw.t16);
 #pragma unroll
@@ -110,16 +180,13 @@ __device__ __forceinline__ void fft512w_inv_a(cd v[4], cd *tile, int lane, const
         v[2 * s] = cadd(a, b);
         v[2 * s + 1] = csub(a, b);
     }
-#pragma unroll
-    for (int j = 0; j < 4; j++) tile[(j >> 1) * 128 + lane + 64 * (j & 1)] = v[j];
+    put_parts(v, tile, lane, half);
 }
 
-__device__ __forceinline__ void fft512w_inv_c(cd v[4], const cd *pair, int lane, int half,
+__device__ __forceinline__ void fft512w_inv_c(cd v[4], const cd *theirs, int lane, int half,
                                               const TwW &tw)
 {
-    const int n0 = lane + 64 * half;
-#pragma unroll
-    for (int k = 0; k < 4; k++) v[k] = pair[(k >> 1) * kLaneTile + (k & 1) * 128 + n0];
+    get_parts(v, theirs, lane, half);
     {
         cd g = tw.beta;
 #pragma unroll
@@ -170,7 +237,7 @@ static_assert(64 * kWaves >= kMaxN0, "one thread per step");
 // 12 waves x 12 KB) and by the chain through the five barriers, about 8,100
 // cycles a step (1,420 / 3,030 / 750 / 1,870 / 1,050 by phase); it is for
 // batches that leave the chip idle.  One MI355X, n0 = 672, up to 256
-// ciphertexts: 2.37-2.5 ms against 4.5-4.6 with the rows one after the other
+// ciphertexts: 2.35-2.5 ms against 4.5-4.6 with the rows one after the other
 // on two waves.  Not kept: the lane exchanges as DPP selects (no LDS traffic,
 // but about 8 cycles an instruction: phase 2 3,950), the first exchange
 // through LDS instead of register swaps (3,970), loading the key words right
@@ -262,11 +329,11 @@ __global__ __launch_bounds__(64 * kWaves) void k_blind_rotate1w2(
             }
 #pragma unroll
             for (int p = 0; p < 4; p++) v[p] = cd{x[2 * p], x[2 * p + 1]};
-            fft512w_fwd_a(v, lds.row[wave & ~1], lane, half, tw);
+            fft512w_fwd_a(v, lds.row[wave ^ 1], lane, half, tw);
         }
         __syncthreads();
         if (is_row) {
-            fft512w_fwd_c(v, lds.row[wave], lane, tw);
+            fft512w_fwd_c(v, lds.row[wave], lane, half, tw);
 #pragma unroll
             for (int q = 0; q < 4; q++) lds.row[wave][q * 64 + lane] = v[q];
         }
@@ -284,14 +351,14 @@ __global__ __launch_bounds__(64 * kWaves) void k_blind_rotate1w2(
 #pragma unroll
             for (int q = 0; q < 4; q++) v[q] = tile[q * 64 + lane];
             wave_lds_sync();
-            fft512w_inv_a(v, tile, lane, tw);
+            fft512w_inv_a(v, tile, lane, half, tw);
         }
         // the next step's key words, in flight until its products
         step = __builtin_amdgcn_readfirstlane(ahead);
         if (step) load_key(step);
         __syncthreads();
         if (!is_row) {
-            fft512w_inv_c(v, lds.col[2 * col], lane, half, tw);
+            fft512w_inv_c(v, lds.col[(wave - kRowWaves) ^ 1], lane, half, tw);
 #pragma unroll
             for (int k = 0; k < 8; k++) {
                 own[k] += trunc_torus32(k & 1 ? v[k >> 1].y : v[k >> 1].x);
