@@ -141,9 +141,9 @@ inline int tuned(const fhe_ctx *ctx, int knob, int B, int dflt)
 // ciphertexts per workgroup (launch_iks21; one MI355X, 64 / 32 / 16: 100
 // ciphertexts 0.20 / 0.15 / 0.15 ms, 256 0.19 / 0.15 / 0.22, 300 0.20 / 0.24 /
 // 0.32, 4096 1.25 / 1.69 / 2.65).  Kinds 10 and 20: workgroups per
-// ciphertext over the digit positions; untuned 8 (one MI355X, n0 = 672, split
-// 1 / 8: kind 10 16 ciphertexts 0.13 / 0.02 ms, 16384 ciphertexts 15.1 /
-// 13.5 ms; kind 20 16384 ciphertexts 31.0 / 28.6 ms).
+// ciphertext over the digit positions; untuned 8, which launch_iks takes as
+// many or few (one MI355X, n0 = 672, split 1 / 8: kind 10 16 ciphertexts 0.13 /
+// 0.02 ms, 4096 ciphertexts 3.73 / 3.38 ms; kind 20 7.67 / 7.19 ms).
 inline int iks_tile(const fhe_ctx *ctx, int kind, int B)
 {
     if (kind == 21) return tuned(ctx, FHE_TUNE_IKS21_TILE, B, B <= 128 ? 16 : B <= 256 ? 32 : 64);

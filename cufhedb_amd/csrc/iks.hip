@@ -102,8 +102,8 @@ __global__ void k_fill_zero32(uint32_t *p, size_t n)
 }
 
 // launch k_iks_rows with NCH = ceil((tn + 1) / 64), tn <= kMaxN0, split
-// ways over the digit positions (1, 2, 4 or 8; a split output is zeroed by a
-// kernel first, so the launch stays capturable)
+// ways over the digit positions (a power of two up to kMaxSplit; a split
+// output is zeroed by a kernel first, so the launch stays capturable)
 template <class TD, int DN, int T, int BB, int NCH = 1>
 void launch_iks_rows(const TD *in, const uint32_t *ksk, uint32_t *out, int tn, int B, int split,
                      hipStream_t s)
@@ -119,6 +119,14 @@ void launch_iks_rows(const TD *in, const uint32_t *ksk, uint32_t *out, int tn, i
     hipLaunchKernelGGL((k_iks_rows<TD, DN, T, BB, NCH>), dim3(B, split), dim3(256), 0, s, in, ksk,
                        out, tn, B);
 }
+
+// A few ciphertexts leave their workgroups waiting for one pair of rows after
+// the other, so they are split further, up to 512 workgroups (one MI355X,
+// n0 = 672, kind 10, split 8 / 16 / 32 / 64, us: 1 ciphertext 19.0 / 12.1 /
+// 8.2 / 6.6, 8 24.6 / 15.4 / 11.2 / 11.5, 32 35.3 / 34.5 / 36.0 / 36.4, 64
+// 64.7 / 66.1 / 66.7 / 68.6; kind 20, 1 36.7 / 20.5 / 12.4 / 8.9, 16 57.0 /
+// 36.5 / 35.6 / 36.6; split 128 is slower again from two ciphertexts on)
+constexpr int kMaxSplit = 64, kSplitWorkgroups = 512;
 
 // Gather form of the same switch for batches that select every key row
 // several times: a workgroup of 1024 threads takes 4096 ciphertexts on a slice
@@ -517,10 +525,13 @@ hipError_t launch_iks(int kind, const void *in, const uint32_t *ksk, uint32_t *o
     switch (kind) {
     case 10:
     case 20: {
-        // `tile` = workgroups per ciphertext over the digit positions; with 8
-        // of them the gather form takes over where it is faster
-        const int split = tile == 2 || tile == 4 || tile == 8 ? tile : 1;
+        // `tile` = workgroups per ciphertext over the digit positions; 8 of
+        // them become more for a few ciphertexts, and the gather form takes
+        // over from 8 where it is faster
+        int split = tile == 2 || tile == 4 || tile == 8 ? tile : 1;
         const bool gather = split == 8 && B >= (kind == 10 ? kGatherFrom10 : kGatherFrom20);
+        if (split == 8)
+            while (split < kMaxSplit && 2 * split * B <= kSplitWorkgroups) split *= 2;
         const auto *x1 = static_cast<const uint32_t *>(in);
         const auto *x2 = static_cast<const uint64_t *>(in);
         if (kind == 10 && gather)

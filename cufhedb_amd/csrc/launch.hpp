@@ -88,8 +88,8 @@ hipError_t launch_sample_extract2(const uint64_t *trlwe, uint64_t *tlwe, int ind
 // kind 10: uint32 domain (dn = 1024), kind 20/21: uint64 domain (dn = 2048)
 // tile: kind 21 (ksk in launch_ksk21_layout's layout), ciphertexts per
 // workgroup: 512 (64), 256 (32) or 128 (else); kinds 10 and 20, workgroups per
-// ciphertext over the digit positions (1, 2, 4, 8; 0 = 1; with 8, large
-// batches take k_iks_gather)
+// ciphertext over the digit positions (1, 2, 4, 8; 0 = 1; with 8, a few
+// ciphertexts take up to 64 and large batches k_iks_gather)
 // ksk of kinds 10 and 20: the reference layout [dn][t][2^basebit - 1][tn + 1]
 // with rows ksk_row_words(tn) words apart, at whole 128-byte lines
 constexpr int ksk_row_words(int tn) { return (tn + 1 + 31) & ~31; }

@@ -1,6 +1,7 @@
 """Key switches 10 and 20 from device rows at whole 128-byte lines
-(csrc/iks.hip): output widths around the lines' 32 words and batches on both
-sides of the gather form's first size, against the oracle (IdentityKeySwitch,
+(csrc/iks.hip): output widths around the lines' 32 words, batches on both sides
+of the gather form's first size, and few enough ciphertexts to be split over
+more workgroups each, against the oracle (IdentityKeySwitch,
 TFHEpp/src/keyswitch.cpp:12-48), word for word.  The keys are random words, so
 a row read from the wrong place shows.
 """
@@ -55,5 +56,26 @@ def test_first_gather_size_kind20():
             got = ctx.iks(20, c[:B])
             for b, w in want.items():
                 assert b >= B or np.array_equal(got[b], w), (B, b)
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("kind", [10, 20])
+def test_few_ciphertexts(kind):
+    """64, 32, 16 and 8 workgroups a ciphertext."""
+    n0, wide = 40, kind == 20
+    n = F.LVL2_N if wide else F.LVL1_N
+    rng = np.random.default_rng(kind + 1)
+    ksk = rng.integers(0, 1 << 32, n * 2 * 1023 * (n0 + 1), np.uint32)
+    ctx = context(n0)
+    try:
+        ctx.load_ksk(kind, ksk)
+        c = rng.integers(0, 1 << (64 if wide else 32), (65, n + 1), np.uint64 if wide else np.uint32)
+        c[0] = 0
+        for B in (1, 2, 8, 9, 16, 17, 32, 33, 65):
+            got = ctx.iks(kind, c[:B])
+            for b in {0, B // 2, B - 1}:
+                want = O.iks64(c[b], ksk, n0, 2, 10) if wide else O.iks32(c[b], ksk, n0)
+                assert np.array_equal(got[b], want), (B, b)
     finally:
         ctx.close()
