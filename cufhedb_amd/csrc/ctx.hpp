@@ -86,8 +86,8 @@ inline hipStream_t pick(fhe_ctx *ctx, void *stream)
 }
 
 // untuned: batches below this many ciphertexts use two waves per polynomial
-// and a compute unit per ciphertext (one MI355X, n0 = 672: 2.4 ms up to 256
-// ciphertexts, 4.9 from 257, where a second round starts; one wave per
+// and a compute unit per ciphertext (one MI355X, n0 = 672: 2.2-2.4 ms up to
+// 256 ciphertexts, 4.5 from 257, where a second round starts; one wave per
 // ciphertext, n0 = 636, 5.17 / 5.41 / 5.94 ms at 256 / 512 / 768).  The two kernels sum in different
 // orders, so moving the line would change the words that a batch returns.
 constexpr int kPbs1TwoWaveBelow = 512;

@@ -431,17 +431,59 @@ __device__ __forceinline__ void transpose_reg_lane_hi_lds(cd v[4], cd *tile, int
     wave_lds_sync();
 }
 
+// Exchange of two registers across lane bit log2(N), N = 4 or 8: lanes with
+// the bit take b of the lane N below into a, lanes without it a of the lane N
+// above into b.  Bank-masked DPP moves at the full rate, three a word with the
+// copy (a select with a DPP operand, two a word, takes about 8 cycles).
+template <int N>
+__device__ __forceinline__ void swap_row_bit(double &a, double &b)
+{
+    constexpr int up = 0x110 + N, down = 0x100 + N;  // row_shr, row_shl
+    constexpr int with = N == 8 ? 0xc : 0xa, without = N == 8 ? 0x3 : 0x5;
+    const uint64_t ua = uint64_t(__double_as_longlong(a)), ub = uint64_t(__double_as_longlong(b));
+    uint32_t w[2][2] = {{uint32_t(ua), uint32_t(ua >> 32)}, {uint32_t(ub), uint32_t(ub >> 32)}};
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const uint32_t x = w[0][k], y = w[1][k];
+        w[0][k] = __builtin_amdgcn_update_dpp(x, y, up, 0xf, with, false);
+        w[1][k] = __builtin_amdgcn_update_dpp(y, x, down, 0xf, without, false);
+    }
+    a = __longlong_as_double((long long)((uint64_t(w[0][1]) << 32) | w[0][0]));
+    b = __longlong_as_double((long long)((uint64_t(w[1][1]) << 32) | w[1][0]));
+}
+
+// 4 x 4 transpose of the register index with lane bits 2-3 (bit 1 of the
+// register with lane bit 3, bit 0 with bit 2).  Its own inverse.
+__device__ __forceinline__ void transpose_reg_lane_mid(cd v[4])
+{
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        swap_row_bit<8>(v[r].x, v[r + 2].x);
+        swap_row_bit<8>(v[r].y, v[r + 2].y);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r += 2) {
+        swap_row_bit<4>(v[r].x, v[r + 1].x);
+        swap_row_bit<4>(v[r].y, v[r + 1].y);
+    }
+}
+
 // 64-point DFT over the lanes of a wave for each of the four register
 // sequences, as three radix-4 passes: the first exchange is the register /
 // lane-bits-4-5 transpose (PERM: lane swaps; otherwise through the tile),
 // the other two go through a wave-private LDS tile of kLaneTile double2
 // (row strides 20 and 5, conflict-free for 16-lane b128 accesses).  The
 // swaps move VALU work in for LDS traffic out, which pays in the blind
-// rotations; both forms move the same words, so the results are identical.
+// rotations.  MID: the second exchange, register / lane bits 2-3, as DPP moves
+// too: 48 of them, about 210 cycles of a SIMD, for four writes and four reads a
+// lane, 72 of the unit that its four SIMDs share, and their round trip (one
+// MI355X, n0 = 672: lvl1 2.35 -> 2.19 ms for one ciphertext, lvl2 5.22 -> 5.00
+// for 61 and 68.5 -> 66.4 for 4096).  All forms move the same words, so the
+// results are identical.
 // t64 = W64^(lane & 15), t16 = W16^(lane & 3).  Input: register r, lane L
 // holds x_r[L]; output: register q, lane l holds X_r[m] for r = l >> 4,
 // m = ((l >> 2) & 3) + 4 (l & 3) + 16 q.
-template <bool PERM, class Tw>
+template <bool PERM, bool MID = false, class Tw>
 __device__ __forceinline__ void lanes64_fwd(cd v[4], cd *tile, int l, Tw t64, Tw t16)
 {
     // T1: (lane L, reg m1) -> lane (L0 = l & 15, m1 = l >> 4), reg L1
@@ -452,12 +494,16 @@ __device__ __forceinline__ void lanes64_fwd(cd v[4], cd *tile, int l, Tw t64, Tw
     dft4<1>(v[0], v[1], v[2], v[3]);
     twiddle4<false>(v, t64);
     // T2: (lane (L0, m1), reg q1) -> lane (L00 = l & 3, rest = l >> 2 = 4 m1 + q1), reg L01
+    if constexpr (MID)
+        transpose_reg_lane_mid(v);
+    else {
 #pragma unroll
-    for (int q1 = 0; q1 < 4; q1++) tile[((l >> 4) * 4 + q1) * 20 + (l & 15)] = v[q1];
-    wave_lds_sync();
+        for (int q1 = 0; q1 < 4; q1++) tile[((l >> 4) * 4 + q1) * 20 + (l & 15)] = v[q1];
+        wave_lds_sync();
 #pragma unroll
-    for (int L01 = 0; L01 < 4; L01++) v[L01] = tile[(l >> 2) * 20 + (l & 3) + 4 * L01];
-    wave_lds_sync();
+        for (int L01 = 0; L01 < 4; L01++) v[L01] = tile[(l >> 2) * 20 + (l & 3) + 4 * L01];
+        wave_lds_sync();
+    }
     dft4<1>(v[0], v[1], v[2], v[3]);
     twiddle4<false>(v, t16);
     // T3: (lane (L00, rest), reg q21) -> lane 4 rest + q21, reg L00
@@ -470,7 +516,7 @@ __device__ __forceinline__ void lanes64_fwd(cd v[4], cd *tile, int l, Tw t64, Tw
     dft4<1>(v[0], v[1], v[2], v[3]);
 }
 
-template <bool PERM, class Tw>
+template <bool PERM, bool MID = false, class Tw>
 __device__ __forceinline__ void lanes64_inv(cd v[4], cd *tile, int l, Tw t64, Tw t16)
 {
     dft4<-1>(v[0], v[1], v[2], v[3]);
@@ -482,12 +528,16 @@ __device__ __forceinline__ void lanes64_inv(cd v[4], cd *tile, int l, Tw t64, Tw
     wave_lds_sync();
     twiddle4<true>(v, t16);
     dft4<-1>(v[0], v[1], v[2], v[3]);
+    if constexpr (MID)
+        transpose_reg_lane_mid(v);
+    else {
 #pragma unroll
-    for (int L01 = 0; L01 < 4; L01++) tile[(l >> 2) * 20 + (l & 3) + 4 * L01] = v[L01];
-    wave_lds_sync();
+        for (int L01 = 0; L01 < 4; L01++) tile[(l >> 2) * 20 + (l & 3) + 4 * L01] = v[L01];
+        wave_lds_sync();
 #pragma unroll
-    for (int q1 = 0; q1 < 4; q1++) v[q1] = tile[((l >> 4) * 4 + q1) * 20 + (l & 15)];
-    wave_lds_sync();
+        for (int q1 = 0; q1 < 4; q1++) v[q1] = tile[((l >> 4) * 4 + q1) * 20 + (l & 15)];
+        wave_lds_sync();
+    }
     twiddle4<true>(v, t64);
     dft4<-1>(v[0], v[1], v[2], v[3]);
     if constexpr (PERM)

@@ -165,7 +165,7 @@ __device__ __forceinline__ void fft512w_fwd_c(cd v[4], cd *tile, int lane, int h
         v[2 * s] = cadd(a, b);
         v[2 * s + 1] = cmul(csub(a, b), tw.t128);
     }
-    lanes64_fwd<true>(v, tile, lane, tw.t64, tw.t16);
+    lanes64_fwd<true, true>(v, tile, lane, tw.t64, tw.t16);
 }
 
 // The inverse (unnormalised: returns 512 z), frequency layout in, time layout
@@ -173,7 +173,7 @@ __device__ __forceinline__ void fft512w_fwd_c(cd v[4], cd *tile, int lane, int h
 // words in the wave's own tile, part C reads the other half's tile.
 __device__ __forceinline__ void fft512w_inv_a(cd v[4], cd *tile, int lane, int half, const TwW &tw)
 {
-    lanes64_inv<true>(v, tile, lane, tw.t64, tw.t16);
+    lanes64_inv<true, true>(v, tile, lane, tw.t64, tw.t16);
 #pragma unroll
     for (int s = 0; s < 2; s++) {
         const cd a = v[2 * s], b = cmulc(v[2 * s + 1], tw.t128);
@@ -233,12 +233,13 @@ static_assert(64 * kWaves >= kMaxN0, "one thread per step");
 // Every value is computed by the same operations in the same order whatever
 // the batch size.
 //
-// Bound by the LDS writes of the row waves (74-80 bytes a clock: phase 2 is
-// 12 waves x 12 KB) and by the chain through the five barriers, about 8,100
-// cycles a step (1,420 / 3,030 / 750 / 1,870 / 1,050 by phase); it is for
+// Bound by the LDS writes of the row waves (74-80 bytes a clock) and by the
+// chain through the five barriers, about 7,500 cycles a step (8,100 with whole
+// exchanges and lane bits 2-3 through LDS: 1,420 / 3,030 / 750 / 1,870 / 1,050
+// by phase); it is for
 // batches that leave the chip idle.  One MI355X, n0 = 672, up to 256
-// ciphertexts: 2.35-2.5 ms against 4.5-4.6 with the rows one after the other
-// on two waves.  Not kept: the lane exchanges as DPP selects (no LDS traffic,
+// ciphertexts: 2.2-2.4 ms against 4.5-4.6 with the rows one after the other
+// on two waves.  Not kept: all lane exchanges as DPP selects (no LDS traffic,
 // but about 8 cycles an instruction: phase 2 3,950), the first exchange
 // through LDS instead of register swaps (3,970), loading the key words right
 // after the products (96 KB through the 64-byte L1 port: phase 3 1,930).

@@ -17,9 +17,12 @@
 //           a radix-4 pass over the registers, then the 64-point DFT over
 //           the lanes as three radix-4 passes: the first exchange by
 //           cross-lane register swaps (v_permlane32_swap /
-//           v_permlane16_swap); the other two by wave-local LDS transposes
-//           (row strides 20 and 5 double2, conflict-free for gfx950's
-//           16-lanes-per-cycle b128 accesses).
+//           v_permlane16_swap), the second by DPP moves, the third by a
+//           wave-local LDS transpose (row stride 5 double2, conflict-free for
+//           gfx950's 16-lanes-per-cycle b128 accesses).  The inverse of a
+//           large batch takes the second through LDS too (row stride 20): the
+//           moves gain nothing there (300 ciphertexts 10.24 against 10.18 ms,
+//           4096 66.8 against 66.4).
 // Layouts: time domain wave w, lane L, register p holds z[L + 64 w + 256 p];
 // frequency domain wave k, lane l, register q holds Z[4 m' + k] with
 // m' = (l >> 4) + 4 ((l >> 2) & 3) + 16 (l & 3) + 64 q.  The inverse runs
@@ -108,7 +111,7 @@ __device__ __forceinline__ void fft1024q_fwd_c(cd v[4], cd *tile, int lane, cons
     // step C: radix-4 over the registers (stride 64), twiddle W256^{L m1}
     dft4<1>(v[0], v[1], v[2], v[3]);
     twiddle4<false>(v, tw.t256);
-    lanes64_fwd<PERM>(v, tile, lane, tw.t64, tw.t16);
+    lanes64_fwd<PERM, PERM>(v, tile, lane, tw.t64, tw.t16);
 }
 
 template <bool PERM = false>
@@ -129,10 +132,10 @@ __device__ __forceinline__ void fft1024q_fwd(cd v[4], cd *xch, int lane, int wav
 // The inverse in two parts around its exchange (words lane + 64 j of the
 // wave's sequence after part A, the wave's words of the four sequences before
 // part C).
-template <bool PERM, class Tw>
+template <bool PERM, bool MID = false, class Tw>
 __device__ __forceinline__ void fft1024q_inv_a(cd v[4], cd *tile, int lane, const Tw &tw)
 {
-    lanes64_inv<PERM>(v, tile, lane, tw.t64, tw.t16);
+    lanes64_inv<PERM, MID>(v, tile, lane, tw.t64, tw.t16);
     twiddle4<true>(v, tw.t256);
     dft4<-1>(v[0], v[1], v[2], v[3]);
 }
@@ -382,10 +385,10 @@ static_assert(64 * kRowWavesQ >= kMaxN0, "one thread per step");
 // run the inverses and update the accumulator.  Each value is computed by the
 // operations of k_blind_rotate2q in the same order.
 //
-// Bound by LDS: about 12,900 of a step's 18,000 cycles move its words (writes
-// at 74-80 bytes a clock), and the transforms' VALU work fills the SIMDs to a
-// similar share.  One MI355X, n0 = 672, up to 256 ciphertexts: 5.2-5.4 ms
-// against 7.9 for k_blind_rotate2q, which has one wave per SIMD there.  Words
+// Bound by LDS (writes at 74-80 bytes a clock) and the transforms' VALU work
+// alike, about 17,200 cycles a step.  One MI355X, n0 = 672, up to 256
+// ciphertexts: 5.0-5.2 ms against 7.9 for k_blind_rotate2q, which has one wave
+// per SIMD there.  Words
 // that stay with their wave in an exchange (one of four) skip LDS; the key
 // loads are spread over the row phases, because issued together they hold the
 // waves up at the L1's 64 bytes a clock (6.3 ms); the powers of the passes'
@@ -520,7 +523,7 @@ __global__ __launch_bounds__(64 * kRowWavesQ) void k_blind_rotate2s(
 #pragma unroll
             for (int q = 0; q < 4; q++) v[q] = tile[q * 64 + lane];
             wave_lds_sync();
-            fft1024q_inv_a<true>(v, tile, lane, tw);
+            fft1024q_inv_a<true, true>(v, tile, lane, tw);
 #pragma unroll
             for (int j = 0; j < 4; j++) tile[lane + 64 * j] = v[j];
         }
@@ -612,9 +615,9 @@ __global__ __launch_bounds__(256) void k_ifft2q(const uint64_t *__restrict__ pol
 }  // namespace
 
 // Up to one ciphertext per compute unit k_blind_rotate2s is faster (one
-// MI355X, n0 = 672: 5.4 against 7.9 ms); beyond, its second round costs as
-// much as k_blind_rotate2q's two or three ciphertexts per unit (10.8 against
-// 10.9 ms at 300, 16.2 against 12.8 at 768), and at the end of a large batch
+// MI355X, n0 = 672: 5.2 against 7.9 ms); beyond, its second round costs as
+// much as k_blind_rotate2q's two or three ciphertexts per unit (10.3 against
+// 10.2 ms at 300, 15.4 against 14.5 at 768), and at the end of a large batch
 // it would replace a part round that costs k_blind_rotate2q only 4.3 ms
 // (4096 against 3840 ciphertexts).
 constexpr int kSmall2q = 256;
