@@ -73,62 +73,67 @@ int prepare_pbs1(fhe_ctx *ctx, hipStream_t s)
 
 int ksk_target(fhe_ctx *ctx, int kind, uint32_t **dst)
 {
+    *dst = nullptr;
+    if (g_capturing) {
+        set_error("key-switching key %d: not during a graph capture", kind);
+        return FHE_ERR_ARG;
+    }
     const size_t words = fhe_ksk_words(&ctx->p, kind);
+    uint32_t *&mem = ctx->ksk_mem[ksk_slot(kind)];
     if (kind == 21) {
-        *dst = nullptr;
         HIP_TRY(hipMalloc(dst, words * sizeof(uint32_t)), "KSK allocation");
+        const hipError_t e = mem ? hipSuccess : hipMalloc(&mem, ksk21_bytes());
+        if (e != hipSuccess) ksk_drop(kind, *dst);
+        HIP_TRY(e, "KSK allocation");
         return FHE_OK;
     }
-    uint32_t *&slot = ctx->ksk[ksk_slot(kind)];
     const int tn = int(ctx->p.n0);
     const size_t spread = words / (tn + 1) * ksk_row_words(tn);
-    if (!slot)
-        HIP_TRY(hipMalloc(&slot, (spread + kKskPadWords) * sizeof(uint32_t)), "KSK allocation");
-    *dst = slot + (spread - words);
+    if (!mem)
+        HIP_TRY(hipMalloc(&mem, (spread + kKskPadWords) * sizeof(uint32_t)), "KSK allocation");
+    *dst = mem + (spread - words);
     return FHE_OK;
+}
+
+void ksk_begin(fhe_ctx *ctx, int kind)
+{
+    if (kind != 21) ctx->ksk[ksk_slot(kind)] = nullptr;
 }
 
 namespace {
 
-// rows of kinds 10 and 20 from the end of the slot's buffer to their places
-int spread_ksk(fhe_ctx *ctx, int kind)
+// rows of kinds 10 and 20 from the end of the key's memory to their places
+hipError_t spread_ksk(fhe_ctx *ctx, int kind)
 {
     const int tn = int(ctx->p.n0);
-    if (ksk_row_words(tn) == tn + 1) return FHE_OK;
+    if (ksk_row_words(tn) == tn + 1) return hipSuccess;
     const size_t rows = fhe_ksk_words(&ctx->p, kind) / (tn + 1), tmp_rows = size_t(1) << 14;
     uint32_t *tmp = nullptr;
     hipError_t e = hipMalloc(&tmp, tmp_rows * (tn + 1) * sizeof(uint32_t));
     if (e == hipSuccess)
-        e = launch_ksk_spread(ctx->ksk[ksk_slot(kind)], tn, rows, tmp, tmp_rows, ctx->stream);
+        e = launch_ksk_spread(ctx->ksk_mem[ksk_slot(kind)], tn, rows, tmp, tmp_rows, ctx->stream);
     const hipError_t es = hipStreamSynchronize(ctx->stream);
-    if (e == hipSuccess) e = es;
     (void)hipFree(tmp);
-    if (e != hipSuccess) {
-        // half moved: not a key any more
-        (void)hipFree(ctx->ksk[ksk_slot(kind)]);
-        ctx->ksk[ksk_slot(kind)] = nullptr;
-    }
-    HIP_TRY(e, "KSK layout");
-    return FHE_OK;
+    return e == hipSuccess ? es : e;
 }
 
 }  // namespace
 
 int ksk_commit(fhe_ctx *ctx, int kind, uint32_t *dst)
 {
-    if (kind != 21) return spread_ksk(ctx, kind);
-    uint32_t *&slot = ctx->ksk[ksk_slot(kind)];
-    uint32_t *to = slot;
-    hipError_t e = to ? hipSuccess : hipMalloc(&to, ksk21_bytes());
-    if (e == hipSuccess) e = launch_ksk21_layout(dst, to, ctx->stream);
-    const hipError_t es = hipStreamSynchronize(ctx->stream);
-    if (e == hipSuccess) e = es;
-    ksk_drop(kind, dst);
-    if (e == hipSuccess)
-        slot = to;
-    else if (to && !slot)
-        (void)hipFree(to);
-    HIP_TRY(e, "KSK 21 layout");
+    const int slot = ksk_slot(kind);
+    hipError_t e;
+    if (kind == 21) {
+        ctx->ksk[slot] = nullptr;
+        e = launch_ksk21_layout(dst, ctx->ksk_mem[slot], ctx->stream);
+        const hipError_t es = hipStreamSynchronize(ctx->stream);
+        if (e == hipSuccess) e = es;
+        ksk_drop(kind, dst);
+    } else {
+        e = spread_ksk(ctx, kind);
+    }
+    HIP_TRY(e, "KSK layout");
+    ctx->ksk[slot] = ctx->ksk_mem[slot];
     return FHE_OK;
 }
 
@@ -221,9 +226,9 @@ int fhe_ctx_destroy(fhe_ctx *ctx)
     if (!ctx) return FHE_OK;
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-    void *bufs[] = {ctx->bk1,  ctx->bk2,    ctx->ksk[0], ctx->ksk[1], ctx->ksk[2],
-                    ctx->trgsw1, ctx->trgsw2, ctx->tv1,  ctx->tv2,    ctx->tmp1,
-                    ctx->tmp0, ctx->tmp2,   ctx->bk1m, ctx->mfma_tab, ctx->bk1w2, ctx->rot2};
+    void *bufs[] = {ctx->bk1,  ctx->bk2,  ctx->trgsw1, ctx->trgsw2,   ctx->tv1, ctx->tv2,
+                    ctx->tmp1, ctx->tmp0, ctx->tmp2,   ctx->bk1m,   ctx->mfma_tab, ctx->bk1w2,
+                    ctx->rot2, ctx->ksk_mem[0], ctx->ksk_mem[1], ctx->ksk_mem[2]};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     for (uint32_t *b : ctx->chain)
@@ -326,6 +331,7 @@ int fhe_load_ksk(fhe_ctx *ctx, int kind, const uint32_t *ksk_host)
     const size_t bytes = fhe_ksk_words(&ctx->p, kind) * sizeof(uint32_t);
     uint32_t *dst = nullptr;
     if (int rc = ksk_target(ctx, kind, &dst)) return rc;
+    ksk_begin(ctx, kind);
     const hipError_t e = hipMemcpy(dst, ksk_host, bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         ksk_drop(kind, dst);

@@ -17,7 +17,11 @@ struct fhe_ctx {
     fhe::cd *bk1 = nullptr;  // lvl01 key, device FD layout
     fhe::cd *bk2 = nullptr;  // lvl02 key, device FD layout
     fhe::cd *rot2 = nullptr; // w2^e, e < 4096: the lvl2 rotation in the frequency domain
-    uint32_t *ksk[3] = {nullptr, nullptr, nullptr};  // kinds 10, 20, 21
+    // kinds 10, 20, 21: the key in service (null: none), and its memory, kept
+    // while a load replaces the key or has failed to (a captured graph may
+    // still name it)
+    uint32_t *ksk[3] = {nullptr, nullptr, nullptr};
+    uint32_t *ksk_mem[3] = {nullptr, nullptr, nullptr};
     fhe::cd *trgsw1 = nullptr;  // external-product TRGSW in device layout
     fhe::cd *trgsw2 = nullptr;
     int variant = FHE_PBS_FP64;
@@ -118,12 +122,15 @@ inline int grow(uint32_t *&buf, size_t &cap, size_t words)
 // discarded).
 constexpr size_t kKskPadWords = 64;
 
-// A key-switching key's way onto the device (capi.hip): ksk_target gives the
-// buffer that receives it in the reference layout (the end of the context's
-// slot; for kind 21 a temporary one), ksk_commit puts it into service (its
-// rows spread to whole lines; kind 21: into the slot in the matrix product's
-// layout) and ksk_drop gives a temporary buffer back without that.
+// A key-switching key's way onto the device (capi.hip).  ksk_target gives the
+// buffer that receives it in the reference layout: the end of the key's own
+// memory, for kind 21 a temporary one.  ksk_begin comes before the first write
+// into it: where that overwrites the key in service, the key goes out of
+// service.  ksk_commit brings the words into the kernels' layout (rows spread to
+// whole lines; kind 21: the matrix product's) and into service; ksk_drop ends
+// a load that failed before.
 int ksk_target(fhe_ctx *ctx, int kind, uint32_t **dst);
+void ksk_begin(fhe_ctx *ctx, int kind);
 int ksk_commit(fhe_ctx *ctx, int kind, uint32_t *dst);
 void ksk_drop(int kind, uint32_t *dst);
 

@@ -138,6 +138,7 @@ int fhe_keygen_ksk_dev(fhe_ctx *ctx, int kind, uint64_t seed, const void *s_dom,
     if (e == hipSuccess)
         e = hipMemcpyAsync(d_noise, noise.data(), records * 4, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) {
+        if (!ksk_dev) ksk_begin(ctx, kind);
         const unsigned grid = unsigned((records + 3) / 4);
         hipLaunchKernelGGL(k_ksk_records, dim3(grid), dim3(256), 0, ctx->stream, seed, g.tag, g.tn,
                            g.t, g.basebit, d_sdom, d_stgt, d_noise, dst, records);

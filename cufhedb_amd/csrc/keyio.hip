@@ -281,8 +281,10 @@ int open_member(File &f, const char *path, int kind, fhe_keyfile_params &q, Memb
 }
 
 // File -> device memory through two pinned staging chunks (disk read of one
-// chunk overlaps the upload of the other).
-int stream_to_device(fhe_ctx *ctx, File &f, void *dst_dev, uint64_t bytes, int elem)
+// chunk overlaps the upload of the other).  `start` runs before the first write
+// into it.
+template <class Fn>
+int stream_to_device(fhe_ctx *ctx, File &f, void *dst_dev, uint64_t bytes, int elem, Fn start)
 {
     constexpr uint64_t kChunk = uint64_t(64) << 20;
     void *pin[2] = {nullptr, nullptr};
@@ -301,6 +303,7 @@ int stream_to_device(fhe_ctx *ctx, File &f, void *dst_dev, uint64_t bytes, int e
         if (e != hipSuccess) break;
         rc = f.read(pin[i], n, elem);
         if (rc != FHE_OK) break;
+        if (off == 0) start();
         e = hipMemcpyAsync(dst + off, pin[i], n, hipMemcpyHostToDevice, ctx->stream);
         if (e == hipSuccess) e = hipEventRecord(done[i], ctx->stream);
         pending[i] = e == hipSuccess;
@@ -322,7 +325,7 @@ int load_ksk_stream(fhe_ctx *ctx, File &f, int ks_kind, uint64_t bytes)
     HIP_TRY(hipSetDevice(ctx->device), "hipSetDevice");
     uint32_t *dst = nullptr;
     if (int rc = ksk_target(ctx, ks_kind, &dst)) return rc;
-    if (int rc = stream_to_device(ctx, f, dst, bytes, 4)) {
+    if (int rc = stream_to_device(ctx, f, dst, bytes, 4, [&] { ksk_begin(ctx, ks_kind); })) {
         ksk_drop(ks_kind, dst);
         return rc;
     }

@@ -119,7 +119,10 @@ void *fhe_ctx_stream(fhe_ctx *ctx);
 enum fhe_bk_format { FHE_BK_INT = 0, FHE_BK_FFT = 1 };
 int fhe_load_bk(fhe_ctx *ctx, int level /* 1 or 2 */, const void *bk_host, int format);
 /* Key-switching key upload (host TFHEpp layout, kind 10/20/21).  The
- * reference keeps these on the host and switches on the CPU. */
+ * reference keeps these on the host and switches on the CPU.  A load that
+ * fails leaves the key that was loaded before, or, once its first words have
+ * been overwritten (kinds 10 and 20 arrive in place), none: a key that did not
+ * arrive whole is never used.  Refused during a graph capture. */
 int fhe_load_ksk(fhe_ctx *ctx, int kind, const uint32_t *ksk_host);
 /* 1 if the context holds a bootstrapping key of `level` (1, 2) / a
  * key-switching key of `kind` (10, 20, 21), else 0.  No reference
