@@ -71,27 +71,23 @@ int prepare_pbs1(fhe_ctx *ctx, hipStream_t s)
     return FHE_OK;
 }
 
-int ksk_target(fhe_ctx *ctx, int kind, uint32_t **dst)
+int ksk_target(fhe_ctx *ctx, int kind, KskLoad &ld)
 {
-    *dst = nullptr;
     if (g_capturing) {
         set_error("key-switching key %d: not during a graph capture", kind);
         return FHE_ERR_ARG;
     }
     const size_t words = fhe_ksk_words(&ctx->p, kind);
+    const size_t tn = size_t(ks_target_n(ctx, kind)), row = size_t(ksk_row_words(int(tn)));
+    const size_t spread = words / (tn + 1) * row;
     uint32_t *&mem = ctx->ksk_mem[ksk_slot(kind)];
-    if (kind == 21) {
-        HIP_TRY(hipMalloc(dst, words * sizeof(uint32_t)), "KSK allocation");
-        const hipError_t e = mem ? hipSuccess : hipMalloc(&mem, ksk21_bytes());
-        if (e != hipSuccess) ksk_drop(kind, *dst);
-        HIP_TRY(e, "KSK allocation");
-        return FHE_OK;
-    }
-    const int tn = int(ctx->p.n0);
-    const size_t spread = words / (tn + 1) * ksk_row_words(tn);
-    if (!mem)
-        HIP_TRY(hipMalloc(&mem, (spread + kKskPadWords) * sizeof(uint32_t)), "KSK allocation");
-    *dst = mem + (spread - words);
+    const size_t mem_bytes = kind == 21 ? ksk21_bytes() : (spread + kKskPadWords) * sizeof(uint32_t);
+    const size_t tmp_words = kind == 21 ? words : row == tn + 1 ? 0 : kSpreadRows * (tn + 1);
+    hipError_t e = tmp_words ? hipMalloc(&ld.tmp, tmp_words * sizeof(uint32_t)) : hipSuccess;
+    if (e == hipSuccess && !mem) e = hipMalloc(&mem, mem_bytes);
+    if (e != hipSuccess) ksk_drop(ld);
+    HIP_TRY(e, "KSK allocation");
+    ld.dst = kind == 21 ? ld.tmp : mem + (spread - words);
     return FHE_OK;
 }
 
@@ -100,46 +96,28 @@ void ksk_begin(fhe_ctx *ctx, int kind)
     if (kind != 21) ctx->ksk[ksk_slot(kind)] = nullptr;
 }
 
-namespace {
-
-// rows of kinds 10 and 20 from the end of the key's memory to their places
-hipError_t spread_ksk(fhe_ctx *ctx, int kind)
+int ksk_commit(fhe_ctx *ctx, int kind, KskLoad &ld)
 {
-    const int tn = int(ctx->p.n0);
-    if (ksk_row_words(tn) == tn + 1) return hipSuccess;
-    const size_t rows = fhe_ksk_words(&ctx->p, kind) / (tn + 1), tmp_rows = size_t(1) << 14;
-    uint32_t *tmp = nullptr;
-    hipError_t e = hipMalloc(&tmp, tmp_rows * (tn + 1) * sizeof(uint32_t));
-    if (e == hipSuccess)
-        e = launch_ksk_spread(ctx->ksk_mem[ksk_slot(kind)], tn, rows, tmp, tmp_rows, ctx->stream);
+    const int slot = ksk_slot(kind), tn = ks_target_n(ctx, kind);
+    uint32_t *mem = ctx->ksk_mem[slot];
+    ctx->ksk[slot] = nullptr;
+    hipError_t e = hipSuccess;
+    if (kind == 21)
+        e = launch_ksk21_layout(ld.dst, mem, ctx->stream);
+    else if (ld.tmp)
+        e = launch_ksk_spread(mem, tn, fhe_ksk_words(&ctx->p, kind) / (tn + 1), ld.tmp, kSpreadRows,
+                              ctx->stream);
     const hipError_t es = hipStreamSynchronize(ctx->stream);
-    (void)hipFree(tmp);
-    return e == hipSuccess ? es : e;
-}
-
-}  // namespace
-
-int ksk_commit(fhe_ctx *ctx, int kind, uint32_t *dst)
-{
-    const int slot = ksk_slot(kind);
-    hipError_t e;
-    if (kind == 21) {
-        ctx->ksk[slot] = nullptr;
-        e = launch_ksk21_layout(dst, ctx->ksk_mem[slot], ctx->stream);
-        const hipError_t es = hipStreamSynchronize(ctx->stream);
-        if (e == hipSuccess) e = es;
-        ksk_drop(kind, dst);
-    } else {
-        e = spread_ksk(ctx, kind);
-    }
-    HIP_TRY(e, "KSK layout");
-    ctx->ksk[slot] = ctx->ksk_mem[slot];
+    ksk_drop(ld);
+    HIP_TRY(e == hipSuccess ? es : e, "KSK layout");
+    ctx->ksk[slot] = mem;
     return FHE_OK;
 }
 
-void ksk_drop(int kind, uint32_t *dst)
+void ksk_drop(KskLoad &ld)
 {
-    if (kind == 21 && dst) (void)hipFree(dst);
+    if (ld.tmp) (void)hipFree(ld.tmp);
+    ld = KskLoad{};
 }
 
 // lvl1 blind rotation (+ sample extraction) with the context's variant
@@ -329,15 +307,15 @@ int fhe_load_ksk(fhe_ctx *ctx, int kind, const uint32_t *ksk_host)
     FHE_CHECK_ARG(slot >= 0, "fhe_load_ksk: kind must be 10, 20 or 21 (got %d)", kind);
     HIP_TRY(hipSetDevice(ctx->device), "hipSetDevice");
     const size_t bytes = fhe_ksk_words(&ctx->p, kind) * sizeof(uint32_t);
-    uint32_t *dst = nullptr;
-    if (int rc = ksk_target(ctx, kind, &dst)) return rc;
+    KskLoad ld;
+    if (int rc = ksk_target(ctx, kind, ld)) return rc;
     ksk_begin(ctx, kind);
-    const hipError_t e = hipMemcpy(dst, ksk_host, bytes, hipMemcpyHostToDevice);
+    const hipError_t e = hipMemcpy(ld.dst, ksk_host, bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
-        ksk_drop(kind, dst);
+        ksk_drop(ld);
         return hip_fail(e, "KSK upload");
     }
-    return ksk_commit(ctx, kind, dst);
+    return ksk_commit(ctx, kind, ld);
 }
 
 int fhe_bk_loaded(const fhe_ctx *ctx, int level)

@@ -122,17 +122,22 @@ inline int grow(uint32_t *&buf, size_t &cap, size_t words)
 // discarded).
 constexpr size_t kKskPadWords = 64;
 
-// A key-switching key's way onto the device (capi.hip).  ksk_target gives the
-// buffer that receives it in the reference layout: the end of the key's own
-// memory, for kind 21 a temporary one.  ksk_begin comes before the first write
-// into it: where that overwrites the key in service, the key goes out of
-// service.  ksk_commit brings the words into the kernels' layout (rows spread to
-// whole lines; kind 21: the matrix product's) and into service; ksk_drop ends
-// a load that failed before.
-int ksk_target(fhe_ctx *ctx, int kind, uint32_t **dst);
+// A key-switching key's way onto the device (capi.hip).  ksk_target allocates
+// all that the load needs and gives the buffer that receives the key in the
+// reference layout: the end of the key's own memory, for kind 21 the temporary
+// one.  ksk_begin comes before the first write into it: where that overwrites
+// the key in service, the key goes out of service.  ksk_commit brings the words
+// into the kernels' layout (rows spread to whole lines; kind 21: the matrix
+// product's) and into service; ksk_drop ends a load that failed before.
+struct KskLoad {
+    uint32_t *dst = nullptr;
+    uint32_t *tmp = nullptr;  // kinds 10 and 20: room for kSpreadRows packed rows; kind 21: dst
+};
+constexpr size_t kSpreadRows = size_t(1) << 14;
+int ksk_target(fhe_ctx *ctx, int kind, KskLoad &ld);
 void ksk_begin(fhe_ctx *ctx, int kind);
-int ksk_commit(fhe_ctx *ctx, int kind, uint32_t *dst);
-void ksk_drop(int kind, uint32_t *dst);
+int ksk_commit(fhe_ctx *ctx, int kind, KskLoad &ld);
+void ksk_drop(KskLoad &ld);
 
 // tuned value of `knob` for a batch of B, or `dflt` if the knob is untuned
 inline int tuned(const fhe_ctx *ctx, int knob, int B, int dflt)

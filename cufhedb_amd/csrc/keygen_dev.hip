@@ -114,9 +114,10 @@ int fhe_keygen_ksk_dev(fhe_ctx *ctx, int kind, uint64_t seed, const void *s_dom,
                   kind);
     HIP_TRY(hipSetDevice(ctx->device), "hipSetDevice");
     const uint64_t records = uint64_t(g.dn) * g.t * ((uint64_t(1) << g.basebit) - 1);
-    uint32_t *dst = ksk_dev;
+    KskLoad ld;
     if (!ksk_dev)
-        if (int rc = ksk_target(ctx, kind, &dst)) return rc;
+        if (int rc = ksk_target(ctx, kind, ld)) return rc;
+    uint32_t *dst = ksk_dev ? ksk_dev : ld.dst;
     // host side: the domain key as 32-bit words (a lvl2 key is 0/1 in 64
     // bits; the host generator truncates the same way) and the noise words
     std::vector<uint32_t> sdom(g.dn);
@@ -149,9 +150,9 @@ int fhe_keygen_ksk_dev(fhe_ctx *ctx, int kind, uint64_t seed, const void *s_dom,
     if (d_sdom) (void)hipFree(d_sdom);
     if (d_stgt) (void)hipFree(d_stgt);
     if (d_noise) (void)hipFree(d_noise);
-    if (e != hipSuccess && !ksk_dev) ksk_drop(kind, dst);
+    if (e != hipSuccess) ksk_drop(ld);
     HIP_TRY(e, "fhe_keygen_ksk_dev");
-    return ksk_dev ? FHE_OK : ksk_commit(ctx, kind, dst);
+    return ksk_dev ? FHE_OK : ksk_commit(ctx, kind, ld);
 }
 
 }  // extern "C"

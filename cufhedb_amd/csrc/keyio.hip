@@ -323,13 +323,13 @@ int stream_to_device(fhe_ctx *ctx, File &f, void *dst_dev, uint64_t bytes, int e
 int load_ksk_stream(fhe_ctx *ctx, File &f, int ks_kind, uint64_t bytes)
 {
     HIP_TRY(hipSetDevice(ctx->device), "hipSetDevice");
-    uint32_t *dst = nullptr;
-    if (int rc = ksk_target(ctx, ks_kind, &dst)) return rc;
-    if (int rc = stream_to_device(ctx, f, dst, bytes, 4, [&] { ksk_begin(ctx, ks_kind); })) {
-        ksk_drop(ks_kind, dst);
+    KskLoad ld;
+    if (int rc = ksk_target(ctx, ks_kind, ld)) return rc;
+    if (int rc = stream_to_device(ctx, f, ld.dst, bytes, 4, [&] { ksk_begin(ctx, ks_kind); })) {
+        ksk_drop(ld);
         return rc;
     }
-    return ksk_commit(ctx, ks_kind, dst);
+    return ksk_commit(ctx, ks_kind, ld);
 }
 
 int load_bk_from_file(fhe_ctx *ctx, File &f, int level, int format, uint64_t bytes, int elem)

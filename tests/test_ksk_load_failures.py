@@ -132,6 +132,20 @@ ctx.close()
 """)
 
 
+@pytest.mark.parametrize("kind", [10, 20, 21])
+def test_reload_without_memory_keeps_the_key(fake, kind):
+    """No room for what the reload needs beside the key's own memory."""
+    run(fake, f"""
+assert load({kind}) == F.FHE_OK
+for how in (load, keygen):
+    fail("hipMalloc", 0)
+    assert how({kind}) == F.FHE_ERR_ALLOC and not fake.fake_pending()
+    assert loaded({kind}) == 1 and switch({kind}) == F.FHE_OK
+ctx.close()
+assert fake.fake_live() == 0
+""")
+
+
 @pytest.mark.parametrize("kind", [10, 21])
 def test_refused_during_capture(fake, kind):
     run(fake, f"""
