@@ -19,6 +19,9 @@ namespace fhe {
 
 namespace {
 
+// workgroups per ciphertext that a few ciphertexts take, at most
+constexpr int kMaxSplit = 64;
+
 // Whole-row form for large bases (kinds 10 and 20: basebit 10, 1023
 // candidate rows per digit position, so ciphertexts rarely share a row): one
 // workgroup per ciphertext, wave w takes every fourth digit position and
@@ -37,7 +40,8 @@ __global__ __launch_bounds__(256) void k_iks_rows(const TD *__restrict__ in,
 {
     constexpr int W = int(sizeof(TD) * 8);
     constexpr int NDIG = DN * T;
-    static_assert(NDIG % 64 == 0, "digit positions are split in multiples of 8 pairs");
+    static_assert(NDIG % (8 * kMaxSplit) == 0,
+                  "every workgroup's range is whole steps of 8 positions at any split");
     constexpr uint32_t mask = (1u << BB) - 1;
     constexpr size_t nd = (size_t(1) << BB) - 1;
     __shared__ uint16_t dig[NDIG];
@@ -126,7 +130,7 @@ void launch_iks_rows(const TD *in, const uint32_t *ksk, uint32_t *out, int tn, i
 // 8.2 / 6.6, 8 24.6 / 15.4 / 11.2 / 11.5, 32 35.3 / 34.5 / 36.0 / 36.4, 64
 // 64.7 / 66.1 / 66.7 / 68.6; kind 20, 1 36.7 / 20.5 / 12.4 / 8.9, 16 57.0 /
 // 36.5 / 35.6 / 36.6; split 128 is slower again from two ciphertexts on)
-constexpr int kMaxSplit = 64, kSplitWorkgroups = 512;
+constexpr int kSplitWorkgroups = 512;
 
 // Gather form of the same switch for batches that select every key row
 // several times: a workgroup of 1024 threads takes 4096 ciphertexts on a slice
