@@ -1,6 +1,7 @@
 // pbs_lvl1w2.hip -- lvl1 blind rotation with two waves per polynomial and the
 // digit rows side by side, for batches too small to fill the GPU with one
-// wave per ciphertext.
+// wave per ciphertext; and with the rows in turn, for larger ones
+// (k_blind_rotate1w2_pair).
 //
 // Same computation as k_blind_rotate1 (pbs_lvl1.hip; TFHEpp BlindRotate,
 // gatebootstrapping.hpp:15-43, CMUX detwfa.cpp:21-30, external product
@@ -29,6 +30,7 @@ namespace {
 constexpr int N1 = Lvl1::N;
 constexpr int kPolyW = 512;  // complex points per polynomial
 constexpr uint32_t kDecOffW = decomp_total_offset<uint32_t, 32, Lvl1::l, Lvl1::Bgbit>();
+constexpr uint32_t kDigitFlipW = (1u << 31) | (1u << 25) | (1u << 19);
 
 // natural frequency of (wave, lane, register) in the output layout
 __host__ __device__ constexpr int f1w(int w, int l, int q)
@@ -135,10 +137,10 @@ __device__ __forceinline__ void get_parts(cd v[4], const cd *tile, int lane, int
 }
 
 // The forward transform of one wave's half, in two parts around the exchange
-// between the two halves (the caller's barrier): part A puts the other half's
-// words into its tile (theirs), part C goes on in the half's own tile, which
-// no other wave touches until the next exchange.
-__device__ __forceinline__ void fft512w_fwd_a(cd v[4], cd *theirs, int lane, int half, const TwW &tw)
+// between the two halves: after part A the caller puts the other half's words
+// into its tile (put_seqs), part C goes on behind the barrier in the half's own
+// tile, which no other wave touches until the next exchange.
+__device__ __forceinline__ void fft512w_fwd_a(cd v[4], const TwW &tw)
 {
     v[1] = cmul(v[1], c8w(1));
     v[2] = cmul(v[2], c8w(2));
@@ -152,7 +154,6 @@ __device__ __forceinline__ void fft512w_fwd_a(cd v[4], cd *theirs, int lane, int
             if (k < 3) g = cmul(g, tw.rho);
         }
     }
-    put_seqs(v, theirs, lane, half);
 }
 
 __device__ __forceinline__ void fft512w_fwd_c(cd v[4], cd *tile, int lane, int half, const TwW &tw)
@@ -330,7 +331,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_blind_rotate1w2(
             }
 #pragma unroll
             for (int p = 0; p < 4; p++) v[p] = cd{x[2 * p], x[2 * p + 1]};
-            fft512w_fwd_a(v, lds.row[wave ^ 1], lane, half, tw);
+            fft512w_fwd_a(v, tw);
+            put_seqs(v, lds.row[wave ^ 1], lane, half);
         }
         __syncthreads();
         if (is_row) {
@@ -381,7 +383,134 @@ __global__ __launch_bounds__(64 * kWaves) void k_blind_rotate1w2(
     }
 }
 
-// one-wave device key -> this kernel's order: slice element (w, q, l) holds
+// gadget digits (trgsw.cpp:21-39) of (X^a acc - acc) at coefficient n, a in
+// [0, 2N), as one signed field extract of the word prepared with the offset and
+// the flipped top bit of every 6-bit field
+__device__ __forceinline__ uint32_t prep_rot(const uint32_t *poly, uint32_t a, int n)
+{
+    const uint32_t idx = (uint32_t(n) - a) & (2u * N1 - 1);
+    uint32_t v = poly[idx & (N1 - 1)];
+    if (idx & N1) v = 0u - v;
+    return (v - poly[n] + kDecOffW) ^ kDigitFlipW;
+}
+__device__ __forceinline__ double digit_w(uint32_t u, int d)
+{
+    const int sh = 32 - Lvl1::Bgbit * (d + 1);
+    return double(int32_t(__builtin_amdgcn_sbfe(int32_t(u), sh, Lvl1::Bgbit)));
+}
+
+// Two waves and 18 KB of LDS per ciphertext, the digit rows one after the
+// other: six ciphertexts fit a compute unit, so batches of more than two rounds
+// of k_blind_rotate1w2's one per unit are faster here (one MI355X, n0 = 672, ms
+// against k_blind_rotate1w2: 513 to 768 ciphertexts 6.4-6.5 / 6.7, 1024 6.9 /
+// 8.9, 4096 25.6 / 35.5, 8192 52.5 / 70.9; up to 256 4.4-4.5 / 2.2, 512 6.5 /
+// 4.5).  The same operations per value in the same order, hence the same words.
+// Three waves per SIMD (166 VGPRs, no spills), bound by the dependence of each
+// transform's passes on each other and two barriers a row.  The lane exchanges
+// as register swaps and DPP moves against all through LDS: 25.6 / 27.5 at 4096,
+// 6.9 / 7.2 at 1024, 6.5 / 6.3 at 600.
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_blind_rotate1w2_pair(
+    const uint32_t *__restrict__ in, int n0, const cd *__restrict__ bk,
+    const uint32_t *__restrict__ tv, int tv_stride, uint32_t *__restrict__ out, int sample_extract,
+    int B)
+{
+    __shared__ uint32_t acc[2][N1];
+    __shared__ cd tiles[2][kLaneTile];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int half = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ct = blockIdx.x;
+    if (ct >= B) return;
+    const uint32_t *c0 = in + size_t(ct) * (n0 + 1);
+    const uint32_t *tvp = tv + size_t(ct) * tv_stride;
+    const TwW tw = make_tww(lane, half);
+    const int nb = lane + 64 * half;
+    cd *own = tiles[half], *theirs = tiles[half ^ 1];
+
+    // acc = (0, X^bbar tv), bbar = 2N - (b >> 21)   (no rounding)
+    {
+        const uint32_t bbar = 2u * N1 - (c0[n0] >> (32 - 1 - Lvl1::nbit));
+#pragma unroll
+        for (int k = 0; k < N1 / 128; k++) {
+            const int n = tid + 128 * k;
+            const uint32_t idx = (uint32_t(n) - bbar) & (2u * N1 - 1);
+            const uint32_t v = tvp[idx & (N1 - 1)];
+            acc[0][n] = 0;
+            acc[1][n] = (idx & N1) ? 0u - v : v;
+        }
+    }
+    __syncthreads();
+
+    constexpr uint32_t kRound = 1u << (32 - 2 - Lvl1::nbit);
+    for (int i = 0; i < n0; i++) {
+        const uint32_t abar = (c0[i] + kRound) >> (32 - 1 - Lvl1::nbit);
+        if (abar == 0) continue;
+        const cd *bki = bk + size_t(i) * (Lvl1::rows * 2 * kPolyW) + half * 256 + lane;
+        cd fd[2][4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) fd[0][q] = fd[1][q] = cd{0.0, 0.0};
+#pragma unroll 1
+        for (int c = 0; c < 2; c++) {
+            uint32_t u[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) u[k] = prep_rot(acc[c], abar, nb + 128 * (k >> 1) + 512 * (k & 1));
+#pragma unroll 1
+            for (int d = 0; d < Lvl1::l; d++) {
+                // key words requested before the transform
+                const cd *k0 = bki + (c * Lvl1::l + d) * 2 * kPolyW;
+                cd b0[4], b1[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    b0[q] = k0[q * 64];
+                    b1[q] = k0[kPolyW + q * 64];
+                }
+                cd v[4];
+#pragma unroll
+                for (int p = 0; p < 4; p++) v[p] = cd{digit_w(u[2 * p], d), digit_w(u[2 * p + 1], d)};
+                fft512w_fwd_a(v, tw);
+                __syncthreads();  // the other wave has left its tile
+                put_seqs(v, theirs, lane, half);
+                __syncthreads();
+                fft512w_fwd_c(v, own, lane, half, tw);
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    cmac(fd[0][q], v[q], b0[q]);
+                    cmac(fd[1][q], v[q], b1[q]);
+                }
+            }
+        }
+        // both waves' rotation reads of acc are complete (the transforms
+        // synchronised them); each wave updates only its own coefficients
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            fft512w_inv_a(fd[c], own, lane, half, tw);
+            __syncthreads();
+            fft512w_inv_c(fd[c], theirs, lane, half, tw);
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const cd z = fd[c][k >> 1];
+                acc[c][nb + 128 * (k >> 1) + 512 * (k & 1)] += trunc_torus32(k & 1 ? z.y : z.x);
+            }
+            // the exchange words are read, and after column 1 the accumulator
+            // is whole
+            __syncthreads();
+        }
+    }
+
+    if (sample_extract) {
+        // SampleExtractIndex 0: out[0] = acc0[0], out[n] = -acc0[N - n], out[N] = acc1[0]
+        uint32_t *o = out + size_t(ct) * (N1 + 1);
+        for (int n = tid; n < N1; n += 128) o[n] = n == 0 ? acc[0][0] : 0u - acc[0][N1 - n];
+        if (tid == 0) o[N1] = acc[1][0];
+    } else {
+        uint32_t *o = out + size_t(ct) * 2 * N1;
+        for (int n = tid; n < N1; n += 128) {
+            o[n] = acc[0][n];
+            o[N1 + n] = acc[1][n];
+        }
+    }
+}
+
+// one-wave device key -> the order of both kernels: slice element (w, q, l) holds
 // frequency f = f1w(w, l, q), which the one-wave layout keeps at register
 // f >> 6 of lane ((f & 7) << 3) | ((f >> 3) & 7)
 __global__ __launch_bounds__(256) void k_bk1_to_w2(const cd *__restrict__ src, cd *__restrict__ dst,
@@ -408,13 +537,22 @@ hipError_t launch_bk1_to_w2(const cd *bk1, cd *bk_w2, int n0, hipStream_t s)
     return hipGetLastError();
 }
 
+// k_blind_rotate1w2 up to two ciphertexts per compute unit, one after the other
+// (its third round makes it the slower one, figures at k_blind_rotate1w2_pair);
+// reached above kPbs1TwoWaveBelow only where a tuned table asks for two waves
+constexpr int kRoundsW2 = 2 * 256;
+
 hipError_t launch_blind_rotate1w2(const uint32_t *in, int n0, const cd *bk, const uint32_t *tv,
                                   int tv_stride, uint32_t *out, bool sample_extract, int B,
                                   hipStream_t s)
 {
     if (B <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_blind_rotate1w2, dim3(B), dim3(64 * kWaves), 0, s, in, n0, bk, tv,
-                       tv_stride, out, int(sample_extract), B);
+    if (B > kRoundsW2)
+        hipLaunchKernelGGL(k_blind_rotate1w2_pair, dim3(B), dim3(128), 0, s, in, n0, bk, tv,
+                           tv_stride, out, int(sample_extract), B);
+    else
+        hipLaunchKernelGGL(k_blind_rotate1w2, dim3(B), dim3(64 * kWaves), 0, s, in, n0, bk, tv,
+                           tv_stride, out, int(sample_extract), B);
     return hipGetLastError();
 }
 

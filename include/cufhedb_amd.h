@@ -362,7 +362,8 @@ enum fhe_tune_knob {
     FHE_TUNE_PBS1_WAVES = 1, /* waves per polynomial of the FP64 lvl1 blind
                                 rotation: 1 (one wave per ciphertext), or 2
                                 (small batches: the digit rows of a CMUX side
-                                by side on one compute unit); untuned: 2
+                                by side on one compute unit, beyond 512
+                                ciphertexts one after the other); untuned: 2
                                 below 512 ciphertexts */
     FHE_TUNE_IKS_SPLIT = 2,  /* workgroups per ciphertext of the lvl1 -> lvl0
                                 key switch (kind 10; 1, 2, 4, 8: the digit
