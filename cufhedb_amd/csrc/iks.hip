@@ -155,11 +155,58 @@ constexpr int kSplitWorkgroups = 512;
 // other (2.7 at 8192, but 64-byte pieces double k_iks_rows' time).
 constexpr int kGatherCols = 16, kGatherPer = 16;  // columns a workgroup, ciphertexts a quad
 constexpr int kGatherTile = 256 * kGatherPer;     // ciphertexts a workgroup
-// from these batches on (kind 10 / 20): one round of the key costs the gather
-// form 1.5-2.1 / 2.8-3.6 ms whatever the batch, k_iks_rows 0.81 / 1.7 us a
-// ciphertext (1800: 1.57 against 1.45 ms, 2000: 1.62 against 1.63; kind 20,
-// 1600: 2.86 against 2.73, 1800: 2.91 against 3.07)
-constexpr int kGatherFrom10 = 2000, kGatherFrom20 = 1700;
+
+// How the gather form splits a batch of B on tn + 1 output columns.
+struct GatherShape {
+    int slices, tiles, split, per;  // split: ranges of `per` digit positions
+    long rounds, cost;              // of workgroups, one a unit; in positions
+};
+
+template <class TD, int DN, int T>
+GatherShape gather_shape(int tn, int B)
+{
+    GatherShape g{};
+    g.slices = (tn + 1 + kGatherCols - 1) / kGatherCols;
+    g.tiles = (B + kGatherTile - 1) / kGatherTile;
+    constexpr int kStep = 16 / int(sizeof(TD)) * T;
+    // splits of the positions, eight at a time (one an XCD), so that the
+    // workgroups fill the 256 compute units (one each), against about three
+    // positions' worth of start and end per workgroup
+    for (int k = 8; k <= 64; k += 8) {
+        const int per = (DN * T / kStep + k - 1) / k * kStep;
+        const long rounds = (long(g.slices) * g.tiles * k + 255) / 256;
+        const long cost = rounds * (per + 3);
+        if (k == 8 || cost < g.cost) g.split = k, g.per = per, g.rounds = rounds, g.cost = cost;
+    }
+    return g;
+}
+
+// Whether B ciphertexts are worth the gather form: a position of one of its
+// rounds costs 3.7 to 5.2 us whatever the batch, k_iks_rows 0.56 ns per
+// 1000 ciphertexts, positions and words of a row, so the line lies where
+// k_iks_rows would read as many words as it can in the gather form's time.
+// Staging a position is slowest when one round holds all workgroups (they all
+// wait for the same positions), and slower when the rows' distance is an even
+// number of lines, more so a multiple of four (they meet in fewer of the
+// memory's channels).  Measured at 30 widths from 31 to 1025 columns, both
+// kinds, 1400 to 2600 ciphertexts; lines by this rule against the crossing (kind
+// 10 / 20): n0 = 255 2299 / 2273 against 2189 / 2331, 511 2273 / 2260 against
+// 2007 / 2151, 636 2020 / 1974 against 1959 / 1941, 672 2030 / 1943 against
+// 1982 / 1747, 1000 1952 / 1941 against 1699 / 1809; at no width of 400 and up is
+// the choice more than 2 % slower than k_iks_rows (one line for all widths, 2000 /
+// 1700: 31 % at n0 = 255, 12 % at 636).  From 2350 ciphertexts on the gather
+// form is the faster one at every width.
+constexpr int kGatherFrom = 2350;
+
+template <class TD, int DN, int T>
+bool gather_pays(int tn, int B)
+{
+    if (B >= kGatherFrom) return true;
+    const GatherShape g = gather_shape<TD, DN, T>(tn, B);
+    const int stride = ksk_row_words(tn), lines = stride / 32;
+    const long unit = g.rounds == 1 ? 9200 : lines % 4 == 0 ? 7900 : lines % 2 == 0 ? 7600 : 6600;
+    return long(B) * stride * (DN * T) >= unit * 1000 * g.cost;
+}
 
 template <class TD, int DN, int T, int BB>
 __global__ __launch_bounds__(1024) void k_iks_gather(const TD *__restrict__ in,
@@ -321,23 +368,11 @@ __global__ __launch_bounds__(256) void k_ksk_spread(const uint32_t *__restrict__
 template <class TD, int DN, int T, int BB>
 void launch_iks_gather(const TD *in, const uint32_t *ksk, uint32_t *out, int tn, int B, hipStream_t s)
 {
-    const int slices = (tn + 1 + kGatherCols - 1) / kGatherCols;
-    const int tiles = (B + kGatherTile - 1) / kGatherTile;
-    constexpr int kStep = 16 / int(sizeof(TD)) * T;
-    auto range = [](int k) { return (DN * T / kStep + k - 1) / k * kStep; };
-    // splits of the positions, eight at a time (one an XCD), so that the
-    // workgroups fill the 256 compute units (one each), against about three
-    // positions' worth of start and end per workgroup
-    int split = 8;
-    long best = 0;
-    for (int k = 8; k <= 64; k += 8) {
-        const long cost = (long(slices) * tiles * k + 255) / 256 * (range(k) + 3);
-        if (k == 8 || cost < best) best = cost, split = k;
-    }
+    const GatherShape g = gather_shape<TD, DN, T>(tn, B);
     const size_t n = size_t(B) * (tn + 1);
     hipLaunchKernelGGL(k_fill_zero32, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, out, n);
-    hipLaunchKernelGGL((k_iks_gather<TD, DN, T, BB>), dim3(unsigned(slices * tiles * split)),
-                       dim3(1024), 0, s, in, ksk, out, tn, B, slices, tiles, range(split));
+    hipLaunchKernelGGL((k_iks_gather<TD, DN, T, BB>), dim3(unsigned(g.slices * g.tiles * g.split)),
+                       dim3(1024), 0, s, in, ksk, out, tn, B, g.slices, g.tiles, g.per);
 }
 
 __global__ void k_tlwe1_lincomb(const uint32_t *__restrict__ a, const uint32_t *__restrict__ b,
@@ -533,7 +568,8 @@ hipError_t launch_iks(int kind, const void *in, const uint32_t *ksk, uint32_t *o
         // them become more for a few ciphertexts, and the gather form takes
         // over from 8 where it is faster
         int split = tile == 2 || tile == 4 || tile == 8 ? tile : 1;
-        const bool gather = split == 8 && B >= (kind == 10 ? kGatherFrom10 : kGatherFrom20);
+        const bool gather = split == 8 && (kind == 10 ? gather_pays<uint32_t, Lvl1::N, KS10::t>(tn, B)
+                                                      : gather_pays<uint64_t, Lvl2::N, KS20::t>(tn, B));
         if (split == 8)
             while (split < kMaxSplit && 2 * split * B <= kSplitWorkgroups) split *= 2;
         const auto *x1 = static_cast<const uint32_t *>(in);

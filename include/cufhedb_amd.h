@@ -369,9 +369,9 @@ enum fhe_tune_knob {
                                 key switch (kind 10; 1, 2, 4, 8: the digit
                                 positions split, sums added with integer
                                 atomics; with 8, up to 64 workgroups for a
-                                few ciphertexts, and batches from 2000 on go
-                                4096 ciphertexts a workgroup, kind 20 from
-                                1700); untuned: 8; needs KSK 10 */
+                                few ciphertexts, and from about 2000 on, the
+                                line depending on n0, 4096 ciphertexts a
+                                workgroup); untuned: 8; needs KSK 10 */
     FHE_TUNE_IKS20_SPLIT = 3 /* the same for the lvl2 -> lvl0 key switch
                                 (kind 20: twice the digit positions, 64-bit
                                 inputs), tuned apart; untuned: 8; needs KSK 20 */
