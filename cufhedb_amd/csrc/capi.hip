@@ -120,6 +120,81 @@ void ksk_drop(KskLoad &ld)
     ld = KskLoad{};
 }
 
+namespace {
+
+// A small batch's kernels take a whole compute unit per ciphertext.  Beside a
+// launch of more than one round on another stream such a workgroup waits for
+// the launch's end, since every place that falls free is too small for it and is
+// filled from the launch; the forms of larger batches get in between.  One
+// MI355X, n0 = 672, ms until the small call is done, alone in a unit / shared:
+// one lvl1 ciphertext beside 1024, 4096 at lvl2 20, 62 / 15, 15; 60 at lvl2
+// beside 1024, 4096 at lvl2 23, 66 / 18, 18; one at lvl1 beside 4096, 16384 at
+// lvl1 23, 80 / 15, 15, 32 24, 84 / 20, 26.  Where the shared form waits as long it
+// is not taken: lvl2 beside lvl1 (86 / 87 ms for 60 beside 16384) and more than a
+// few ciphertexts of lvl1 beside lvl1 (60: 83 / 87 in all).
+// The matrix-core and gather key switches need a unit too and wait: 100 rows of
+// kind 21 beside 4096 at lvl2 57 ms, 14 in the column-per-lane form they
+// replaced, but both together 60 against 75.
+constexpr int kLongLvl1 = 2048, kLongLvl2 = 768;  // ciphertexts of one round
+constexpr int kFewLvl1 = 32;
+
+// a status that is no failure of the call under way: nothing that the next
+// launch's check should find
+void forget(hipError_t e)
+{
+    if (e != hipSuccess && hipPeekAtLastError() == e) (void)hipGetLastError();
+}
+
+// clears what has come to its end
+void refresh(fhe_ctx::LongRotation &l)
+{
+    if (!l.levels) return;
+    // a question only, whatever capture any thread may have open
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const hipError_t e = hipEventQuery(l.done);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipErrorNotReady) l.levels = 0;
+    forget(e);
+}
+
+// the rotation of B ciphertexts just launched on s
+void note_long(fhe_ctx *ctx, int level, int B, hipStream_t s)
+{
+    if (B <= (level == 1 ? kLongLvl1 : kLongLvl2)) return;
+    // a captured launch runs later, if ever
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    const hipError_t ec = hipStreamIsCapturing(s, &cap);
+    if (ec != hipSuccess || cap != hipStreamCaptureStatusNone) return forget(ec);
+    std::lock_guard<std::mutex> lk(ctx->longs_mu);
+    fhe_ctx::LongRotation *at = nullptr;
+    for (auto &l : ctx->longs) {
+        refresh(l);
+        if (!l.levels ? !at : l.stream == s) at = &l;
+    }
+    if (!at) return;
+    at->stream = s;
+    const hipError_t er = hipEventRecord(at->done, s);
+    at->levels = er == hipSuccess ? at->levels | level : 0;
+    forget(er);
+}
+
+// levels (bits as in LongRotation) of the long rotations that another stream
+// than s still has in flight
+int beside_long(fhe_ctx *ctx, hipStream_t s)
+{
+    std::lock_guard<std::mutex> lk(ctx->longs_mu);
+    int levels = 0;
+    for (auto &l : ctx->longs) {
+        if (l.stream == s) continue;
+        refresh(l);
+        levels |= l.levels;
+    }
+    return levels;
+}
+
+}  // namespace
+
 // lvl1 blind rotation (+ sample extraction) with the context's variant
 int launch_pbs1(fhe_ctx *ctx, const uint32_t *in, const uint32_t *tv, int tv_stride,
                 uint32_t *out, bool se, int B, hipStream_t s)
@@ -131,16 +206,28 @@ int launch_pbs1(fhe_ctx *ctx, const uint32_t *in, const uint32_t *tv, int tv_str
         HIP_TRY(launch_blind_rotate1_mfma(in, n0, ctx->bk1m, ctx->mfma_tab, tv, tv_stride, out, se,
                                           B, s),
                 "pbs lvl01 (split MFMA)");
-        return FHE_OK;
-    }
-    if (pbs1_waves(ctx, B) == 2) {
+    } else if (pbs1_waves(ctx, B) == 2) {
         int rc = prepare_pbs1(ctx, s);
         if (rc) return rc;
-        HIP_TRY(launch_blind_rotate1w2(in, n0, ctx->bk1w2, tv, tv_stride, out, se, B, s),
+        const int beside = beside_long(ctx, s);
+        const bool shared = (beside & 2) || ((beside & 1) && B <= kFewLvl1);
+        HIP_TRY(launch_blind_rotate1w2(in, n0, ctx->bk1w2, tv, tv_stride, out, se, B, s, shared),
                 "pbs lvl01 (two waves per polynomial)");
-        return FHE_OK;
+    } else {
+        HIP_TRY(launch_blind_rotate1(in, n0, ctx->bk1, tv, tv_stride, out, se, B, s), "pbs lvl01");
     }
-    HIP_TRY(launch_blind_rotate1(in, n0, ctx->bk1, tv, tv_stride, out, se, B, s), "pbs lvl01");
+    note_long(ctx, 1, B, s);
+    return FHE_OK;
+}
+
+int launch_pbs2(fhe_ctx *ctx, const uint32_t *in, const uint64_t *tv, int tv_stride, uint64_t *out,
+                bool se, int B, hipStream_t s, const char *what, int tv_period)
+{
+    const bool shared = beside_long(ctx, s) & 2;
+    HIP_TRY(launch_blind_rotate2q(in, int(ctx->p.n0), ctx->bk2, ctx->rot2, tv, tv_stride, out, se, B, s,
+                                  tv_period, shared),
+            what);
+    note_long(ctx, 2, B, s);
     return FHE_OK;
 }
 
@@ -184,6 +271,8 @@ int fhe_ctx_create(const fhe_params *p, int device, fhe_ctx **out)
     hipError_t e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreate(&ctx->ev0);
     if (e == hipSuccess) e = hipEventCreate(&ctx->ev1);
+    for (auto &l : ctx->longs)
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&l.done, hipEventDisableTiming);
     if (e == hipSuccess) e = hipMalloc(&ctx->tv1, Lvl1::N * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMalloc(&ctx->tv2, Lvl2::N * sizeof(uint64_t));
     if (e != hipSuccess) {
@@ -217,6 +306,8 @@ int fhe_ctx_destroy(fhe_ctx *ctx)
         if (b) (void)hipFree(b);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
+    for (auto &l : ctx->longs)
+        if (l.done) (void)hipEventDestroy(l.done);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return FHE_OK;
@@ -366,10 +457,7 @@ int fhe_pbs_lvl02_dev(fhe_ctx *ctx, const uint32_t *in_dev, const uint64_t *tv_d
         set_error("fhe_pbs_lvl02_dev: lvl02 bootstrapping key not loaded");
         return FHE_ERR_NOT_LOADED;
     }
-    HIP_TRY(launch_blind_rotate2q(in_dev, int(ctx->p.n0), ctx->bk2, ctx->rot2, tv_dev, tv_stride, out_dev, true,
-                                 B, pick(ctx, stream)),
-            "pbs lvl02");
-    return FHE_OK;
+    return launch_pbs2(ctx, in_dev, tv_dev, tv_stride, out_dev, true, B, pick(ctx, stream), "pbs lvl02");
 }
 
 int fhe_blind_rotate_lvl02_dev(fhe_ctx *ctx, const uint32_t *in_dev, const uint64_t *tv_dev,
@@ -382,10 +470,8 @@ int fhe_blind_rotate_lvl02_dev(fhe_ctx *ctx, const uint32_t *in_dev, const uint6
         set_error("fhe_blind_rotate_lvl02_dev: lvl02 bootstrapping key not loaded");
         return FHE_ERR_NOT_LOADED;
     }
-    HIP_TRY(launch_blind_rotate2q(in_dev, int(ctx->p.n0), ctx->bk2, ctx->rot2, tv_dev, tv_stride, acc_dev,
-                                 false, B, pick(ctx, stream)),
-            "blind rotate lvl02");
-    return FHE_OK;
+    return launch_pbs2(ctx, in_dev, tv_dev, tv_stride, acc_dev, false, B, pick(ctx, stream),
+                       "blind rotate lvl02");
 }
 
 int fhe_sample_extract_lvl1_dev(fhe_ctx *ctx, const uint32_t *trlwe_dev, uint32_t *tlwe_dev,
@@ -547,9 +633,9 @@ int run_bootstrap(fhe_ctx *ctx, int in_level, const void *in, int out_level, voi
         HIP_TRY(tv.ide ? launch_tv_ide<uint64_t>(ctx->tv2, uint32_t(tv.value), Lvl2::N, s)
                        : launch_tv_const<uint64_t>(ctx->tv2, tv.value, Lvl2::N, s),
                 "test vector");
-        HIP_TRY(launch_blind_rotate2q(tmp0, n0, ctx->bk2, ctx->rot2, ctx->tv2, 0,
-                                     static_cast<uint64_t *>(out), true, B, s),
-                "pbs lvl02");
+        if (int rc = launch_pbs2(ctx, tmp0, ctx->tv2, 0, static_cast<uint64_t *>(out), true, B, s,
+                                 "pbs lvl02"))
+            return rc;
         if (post)
             HIP_TRY(launch_tlwe_add_body<uint64_t>(static_cast<uint64_t *>(out), Lvl2::N + 1, post,
                                                    B, s),

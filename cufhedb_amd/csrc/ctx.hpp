@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 
 #include "common.hpp"
 #include "fft64.hpp"
@@ -66,6 +67,15 @@ struct fhe_ctx {
     int tune_batch[kTuneKnobs][kTuneMax] = {};
     int tune_val[kTuneKnobs][kTuneMax] = {};
     int tune_n[kTuneKnobs] = {};
+    // blind rotations of more than one round last launched on up to kLong
+    // streams, which small batches beside them ask for (beside_long)
+    static constexpr int kLong = 4;
+    struct LongRotation {
+        hipEvent_t done = nullptr;
+        hipStream_t stream = nullptr;
+        int levels = 0;  // bit 0: lvl1, bit 1: lvl2; 0: none in flight
+    } longs[kLong];
+    std::mutex longs_mu;
 };
 
 namespace fhe {
@@ -173,6 +183,9 @@ inline int pbs1_waves(const fhe_ctx *ctx, int B)
 int launch_pbs1(fhe_ctx *ctx, const uint32_t *in, const uint32_t *tv, int tv_stride,
                 uint32_t *out, bool se, int B, hipStream_t s);
 int prepare_pbs1(fhe_ctx *ctx, hipStream_t s);
+// the same at lvl2; tv_period as in launch_blind_rotate2q
+int launch_pbs2(fhe_ctx *ctx, const uint32_t *in, const uint64_t *tv, int tv_stride, uint64_t *out,
+                bool se, int B, hipStream_t s, const char *what, int tv_period = 0);
 
 // Buffers a lvl1 gate bootstrap works in: B lvl1 TLWEs (the gate's linear
 // combination), B lvl0 TLWEs (after the key switch) and one test vector.

@@ -46,11 +46,13 @@ hipError_t launch_sample_extract1(const uint32_t *trlwe, uint32_t *tlwe, int ind
 
 // ---- lvl1, two waves per polynomial, rows in parallel (small batches),
 // pbs_lvl1w2.hip
-// key: the one-wave device key with each (i, row, col) slice permuted
+// key: the one-wave device key with each (i, row, col) slice permuted.
+// shared: the compute units are busy with another launch (the form that does
+// not need one of its own, at any batch size; the words are the same)
 hipError_t launch_bk1_to_w2(const cd *bk1, cd *bk_w2, int n0, hipStream_t s);
 hipError_t launch_blind_rotate1w2(const uint32_t *in, int n0, const cd *bk, const uint32_t *tv,
                                   int tv_stride, uint32_t *out, bool sample_extract, int B,
-                                  hipStream_t s);
+                                  hipStream_t s, bool shared = false);
 
 // ---- lvl1 split-MFMA variant, pbs_lvl1_mfma.hip -------------------------
 size_t mfma_tables_bytes();
@@ -69,10 +71,12 @@ hipError_t launch_blind_rotate1_mfma(const uint32_t *in, int n0, const float *bk
 size_t bk2q_device_elems(int n0);
 hipError_t launch_bk2q_from_int(const uint64_t *bk_int, cd *bk_dev, int n0, hipStream_t s);
 // tv_period > 0: ciphertext c uses test vector c % tv_period (tv_stride apart).
-// rot: the table of launch_rot2q_table (w2^e, e < 4096)
+// rot: the table of launch_rot2q_table (w2^e, e < 4096).  shared: as for
+// launch_blind_rotate1w2
 hipError_t launch_blind_rotate2q(const uint32_t *in, int n0, const cd *bk, const cd *rot,
                                  const uint64_t *tv, int tv_stride, uint64_t *out,
-                                 bool sample_extract, int B, hipStream_t s, int tv_period = 0);
+                                 bool sample_extract, int B, hipStream_t s, int tv_period = 0,
+                                 bool shared = false);
 size_t rot2q_elems();
 hipError_t launch_rot2q_table(cd *rot, hipStream_t s);
 hipError_t launch_ifft2q(const uint64_t *poly, double *fd, int B, hipStream_t s);

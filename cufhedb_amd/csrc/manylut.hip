@@ -153,9 +153,8 @@ int fhe_pbs_many_lut_lvl02_dev(fhe_ctx *ctx, const uint32_t *in_dev, const uint6
     rc = many_scratch(ctx, 1, size_t(B) * 2 * Lvl2::N * 2, &acc32);
     if (rc) return rc;
     uint64_t *acc = reinterpret_cast<uint64_t *>(acc32);
-    HIP_TRY(launch_blind_rotate2q(rounded, int(ctx->p.n0), ctx->bk2, ctx->rot2, tv_dev, tv_stride,
-                                  acc, false, B, s),
-            "blind rotate lvl02");
+    rc = launch_pbs2(ctx, rounded, tv_dev, tv_stride, acc, false, B, s, "blind rotate lvl02");
+    if (rc) return rc;
     const size_t total = size_t(B) * num_out * (Lvl2::N + 1);
     hipLaunchKernelGGL((k_extract_many<uint64_t, Lvl2::N>), dim3(blocks(total)), dim3(256), 0, s,
                        acc, out_dev, num_out, total);

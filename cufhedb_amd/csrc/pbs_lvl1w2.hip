@@ -544,10 +544,10 @@ constexpr int kRoundsW2 = 2 * 256;
 
 hipError_t launch_blind_rotate1w2(const uint32_t *in, int n0, const cd *bk, const uint32_t *tv,
                                   int tv_stride, uint32_t *out, bool sample_extract, int B,
-                                  hipStream_t s)
+                                  hipStream_t s, bool shared)
 {
     if (B <= 0) return hipSuccess;
-    if (B > kRoundsW2)
+    if (shared || B > kRoundsW2)
         hipLaunchKernelGGL(k_blind_rotate1w2_pair, dim3(B), dim3(128), 0, s, in, n0, bk, tv,
                            tv_stride, out, int(sample_extract), B);
     else

@@ -633,10 +633,11 @@ hipError_t launch_bk2q_from_int(const uint64_t *bk_int, cd *bk_dev, int n0, hipS
 
 hipError_t launch_blind_rotate2q(const uint32_t *in, int n0, const cd *bk, const cd *rot,
                                  const uint64_t *tv, int tv_stride, uint64_t *out,
-                                 bool sample_extract, int B, hipStream_t s, int tv_period)
+                                 bool sample_extract, int B, hipStream_t s, int tv_period,
+                                 bool shared)
 {
     if (B <= 0) return hipSuccess;
-    if (B <= kSmall2q)
+    if (!shared && B <= kSmall2q)
         hipLaunchKernelGGL(k_blind_rotate2s, dim3(B), dim3(64 * kRowWavesQ), 0, s, in, n0, bk, rot,
                            tv, tv_stride, tv_period, out, int(sample_extract));
     else
