@@ -221,9 +221,10 @@ def operator_context(F, which=None):
 
 
 TUNE = {
-    "iks21_tile": ("ciphertexts per workgroup of the lvl2 -> lvl1 key switch",
+    "iks21_tile": ("tile of the lvl2 -> lvl1 key switch (8, 16: 128 ciphertexts a workgroup, "
+                   "32: 256, 64: 512)",
                    (32, 128, 512, 1024, 2048, 4096, 16384)),
-    "pbs1_waves": ("waves per ciphertext of the lvl1 blind rotation",
+    "pbs1_waves": ("waves per polynomial of the lvl1 blind rotation",
                    (64, 256, 512, 1024, 2048)),
     "iks_split": ("workgroups per ciphertext of the lvl1 -> lvl0 key switch",
                   (16, 64, 256, 1024, 4096, 16384)),
@@ -237,7 +238,7 @@ KNOBS = (("iks21_tile", "TUNE_IKS21_TILE"), ("pbs1_waves", "TUNE_PBS1_WAVES"),
 def autotune(F, ctx):
     """Shapes measured on this GPU per batch size and kept in the context for
     the query pipelines: the lvl2 -> lvl1 key switch's tile, the lvl1 blind
-    rotation's waves per ciphertext and the lvl1 -> lvl0 and lvl2 -> lvl0
+    rotation's waves per polynomial and the lvl1 -> lvl0 and lvl2 -> lvl0
     key switches' workgroups per ciphertext (each tuned on its own key)."""
     out = {}
     for name, attr in KNOBS:

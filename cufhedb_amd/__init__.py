@@ -433,7 +433,7 @@ class Context:
         """Time every candidate of `knob` (TUNE_IKS21_TILE: ciphertexts per
         workgroup of the lvl2 -> lvl1 key switch, 8 and 16 standing for 128,
         32 for 256 and 64 for 512, needs KSK 21;
-        TUNE_PBS1_WAVES: waves per ciphertext of the lvl1 blind rotation,
+        TUNE_PBS1_WAVES: waves per polynomial of the lvl1 blind rotation,
         needs BK lvl01; TUNE_IKS_SPLIT / TUNE_IKS20_SPLIT: workgroups per
         ciphertext of the lvl1 -> lvl0 / lvl2 -> lvl0 key switch, needs KSK
         10 / 20) at each batch size and keep the fastest; returns

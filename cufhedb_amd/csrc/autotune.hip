@@ -3,11 +3,11 @@
 // The reference has nothing to tune: it launches one ciphertext per call
 // (src/cuHEDB/fft_gpu/cufft_gpu.cuh:250-271).  Batched, the lvl2 -> lvl1
 // key switch has a real trade-off: a workgroup switching C ciphertexts reads
-// each selected key row once for all C of them (less L2 / Infinity Cache
-// traffic per ciphertext), while a small batch split into few tiles leaves
-// compute units idle; the FP64 lvl1 blind rotation can give a ciphertext one
-// wave or two (two finish a small batch sooner, one uses the GPU best once
-// the batch fills it).  fhe_autotune times every candidate of a knob on the
+// each key block once for all C of them (less L2 / Infinity Cache traffic per
+// ciphertext), while a small batch leaves most of a large tile empty (of its
+// knob's values 8 and 16 are the same kernel); the FP64 lvl1 blind rotation can
+// give a ciphertext one wave, or two waves per polynomial (which finish a small
+// batch sooner; one uses the GPU best once the batch fills it).  fhe_autotune times every candidate of a knob on the
 // context's own keys at each requested batch size and keeps the fastest per
 // size in the context.  The key-switch candidates compute the same integers;
 // the blind-rotation candidates decrypt identically (different FP64

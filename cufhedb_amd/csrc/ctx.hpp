@@ -100,10 +100,11 @@ inline hipStream_t pick(fhe_ctx *ctx, void *stream)
 }
 
 // untuned: batches below this many ciphertexts use two waves per polynomial
-// and a compute unit per ciphertext (one MI355X, n0 = 672: 2.2-2.4 ms up to
-// 256 ciphertexts, 4.5 from 257, where a second round starts; one wave per
-// ciphertext, n0 = 636, 5.17 / 5.41 / 5.94 ms at 256 / 512 / 768).  The two kernels sum in different
-// orders, so moving the line would change the words that a batch returns.
+// and a compute unit per ciphertext (one MI355X, n0 = 672: 2.2 ms up to 256
+// ciphertexts, 4.5 from 257, where a second round starts, 6.5 beyond 512; one
+// wave per ciphertext 5.4 / 5.7 / 6.1 ms at 256 / 512 / 768).  The two kernels
+// sum in different orders, so moving the line would change the words that a
+// batch returns.
 constexpr int kPbs1TwoWaveBelow = 512;
 
 // set on this thread between fhe_graph_begin and fhe_graph_end: scratch
@@ -163,9 +164,10 @@ inline int tuned(const fhe_ctx *ctx, int knob, int B, int dflt)
 // ciphertexts per workgroup (launch_iks21; one MI355X, 64 / 32 / 16: 100
 // ciphertexts 0.20 / 0.15 / 0.15 ms, 256 0.19 / 0.15 / 0.22, 300 0.20 / 0.24 /
 // 0.32, 4096 1.25 / 1.69 / 2.65).  Kinds 10 and 20: workgroups per
-// ciphertext over the digit positions; untuned 8, which launch_iks takes as
-// many or few (one MI355X, n0 = 672, split 1 / 8: kind 10 16 ciphertexts 0.13 /
-// 0.02 ms, 4096 ciphertexts 3.73 / 3.38 ms; kind 20 7.67 / 7.19 ms).
+// ciphertext over the digit positions; untuned 8, with which launch_iks takes
+// more for a few ciphertexts and the gather form for large batches (one MI355X,
+// n0 = 672, 1 / 8: kind 10 16 ciphertexts 0.14 / 0.015 ms, 1024 0.88 / 0.84,
+// 4096 3.65 / 2.12; kind 20 0.31 / 0.03, 1.82 / 1.75, 7.35 / 3.61).
 inline int iks_tile(const fhe_ctx *ctx, int kind, int B)
 {
     if (kind == 21) return tuned(ctx, FHE_TUNE_IKS21_TILE, B, B <= 128 ? 16 : B <= 256 ? 32 : 64);

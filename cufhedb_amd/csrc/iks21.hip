@@ -7,7 +7,8 @@
 // a product of a one-hot matrix (ciphertexts x 8 slots per position) with the
 // key.  The key's 32-bit words are split into four signed bytes (their sum
 // with weights 2^8l is the word mod 2^32), which makes it an int8 product with
-// exact 32-bit sums: |sum| <= 20480 * 128 < 2^31.
+// exact 32-bit sums: a position selects at most two of the bytes, |sum| <=
+// 2 * 20480 * 128 < 2^31.
 //
 // v_smfmac_i32_32x32x64_i8 multiplies a 2:4-sparse left operand at twice the
 // dense rate, and one-hot digits are sparse: a position's eight slots are two

@@ -207,7 +207,7 @@ constexpr int kColWaves = 4;                  // two halves per accumulator colu
 constexpr int kWaves = kRowWaves + kColWaves; // 16: also (column, half, register) of the products
 static_assert(kWaves == 2 * 2 * 4, "one product wave per column, half and register");
 
-// LDS of one blind rotation (106 KB of the CU's 160).  ext holds a column
+// LDS of one blind rotation (108 KB of the CU's 160).  ext holds a column
 // followed by its negation and the column again, so that coefficient n of
 // X^a acc is word ((n - a) mod 2N) + k with the wrap's sign in the data and
 // the lane's eight words at immediate offsets from one base.
@@ -239,7 +239,7 @@ static_assert(64 * kWaves >= kMaxN0, "one thread per step");
 // exchanges and lane bits 2-3 through LDS: 1,420 / 3,030 / 750 / 1,870 / 1,050
 // by phase); it is for
 // batches that leave the chip idle.  One MI355X, n0 = 672, up to 256
-// ciphertexts: 2.2-2.4 ms against 4.5-4.6 with the rows one after the other
+// ciphertexts: 2.2 ms against 4.5-4.6 with the rows one after the other
 // on two waves.  Not kept: all lane exchanges as DPP selects (no LDS traffic,
 // but about 8 cycles an instruction: phase 2 3,950), the first exchange
 // through LDS instead of register swaps (3,970), loading the key words right
